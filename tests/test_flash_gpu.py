@@ -103,6 +103,35 @@ def test_tail_window_n_is_dense_causal_rows(dtype, heads, dev):
     _check(out, ref, "tail_split")
 
 
+@pytest.mark.parametrize("t,n,front,window,noncausal", [
+    (2, 257, 0, 257, True), (65, 1023, 0, 1023, True), (1, 4099, 0, 4099, True),  # a handful of tiles; one row
+    (300, 700, 0, 700, False), (130, 2049, 0, 2049, False),  # causal rows that end inside and before later chunks
+    (64, 9000, 70, 3000, False),                             # chunks between the front and the window hold nothing
+    (33, 5000, 0, 1000, False)])
+@pytest.mark.parametrize("heads,d", [((32, 8), 128), ((8, 4), 128), ((4, 4), 128), ((8, 2), 64)],
+                         ids=["gqa4", "gqa2", "mha", "d64"])
+def test_split_chunks(t, n, front, window, noncausal, heads, d, dev):
+    """Few rows over many keys: the key range is cut into chunks down to 4 tiles and merged; against float64."""
+    print(f"case split_chunks t={t} n={n} front={front} window={window} {noncausal} {heads} d={d}", flush=True)
+    from bigger_bird_amd import exact_attention
+
+    H, Hkv = heads
+    q, k, v = _rand((H, t, d), 41), _rand((Hkv, n, d), 42), _rand((Hkv, n, d), 43)
+    kw = dict(num_heads=H, kv_groups=H // Hkv, scale=d ** -0.5)
+    if noncausal:
+        out = exact_attention(q.to(dev), k.to(dev), v.to(dev), **kw)
+        mask = torch.ones(t, n, dtype=torch.bool)
+    else:
+        none = torch.empty(H, 1, 0, dtype=torch.int32, device=dev)
+        out = bigger_bird_flash(q.to(dev), k.to(dev), v.to(dev), none, front=front, window=window, **kw)
+        rows, keys = torch.arange(n - t, n)[:, None], torch.arange(n)[None]
+        mask = (keys <= rows) & ((keys < front) | (keys > rows - window))
+    ref = torch.nn.functional.scaled_dot_product_attention(
+        q.double()[None], k.double().repeat_interleave(H // Hkv, 0)[None],
+        v.double().repeat_interleave(H // Hkv, 0)[None], attn_mask=mask, scale=d ** -0.5)[0]
+    _check(out, ref, "split_chunks")
+
+
 def test_full_budget_equals_dense_causal(dev):
     """modal_rd/selfcheck.py:36-41: routing every column outside sink/window gives exact causal attention."""
     print("case full_budget", flush=True)

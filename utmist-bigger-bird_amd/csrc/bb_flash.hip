@@ -164,6 +164,7 @@ __global__ __launch_bounds__(64 * NW, 1) void flash_kernel(FlashParams p) {
   const int64_t qw0 = p.offset + rw * p.pos_step;
   const int64_t qw1 = p.offset + (rw + RW - 1 < r1 ? rw + RW - 1 : r1) * p.pos_step;
   const uint8_t* km = HAS_MASK ? p.key_mask + (int64_t)batch * p.smb : nullptr;
+  if (SPLIT && chunk_unused(p, chunk, qlo, qhi)) return;  // the merge skips it
 
   WaveState<D, QB> st;
 #pragma unroll
@@ -358,7 +359,10 @@ __global__ __launch_bounds__(64 * NW, 1) void flash_kernel(FlashParams p) {
   }
 }
 
-// Combine split partials: one wave per (head, row); lanes cover D.
+// Combine split partials: one wave per (head, row); lanes cover D. Chunks that hold no key of the row are skipped (the
+// split kernels write none for a workgroup of such rows). The chunks' (max, sum) pairs are read by
+// one lane each, 64 at a time, and the partial rows eight at a time, so the latency is that of a few round trips and
+// does not grow with the chunk count.
 template <bool F16, int D>
 __global__ __launch_bounds__(256) void flash_merge_kernel(FlashParams p) {
   const int64_t item = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -367,27 +371,48 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashParams p) {
   if (item >= (int64_t)p.BH * rows) return;
   const int bh = (int)(item / rows);
   const int64_t row = item % rows;
-  float M = -1.0e30f;
-  for (int c = 0; c < p.n_chunks; ++c) {
-    const int64_t base = ((int64_t)c * p.BH + bh) * p.T + row;
-    M = fmaxf(M, p.part_ml[2 * base]);
-  }
-  float L = 0.0f;
-  constexpr int PER = (D + 63) / 64;
-  float acc[PER];
+  const int64_t q = p.offset + row * p.pos_step;
+  const int64_t base0 = (int64_t)bh * p.T + row, bstep = (int64_t)p.BH * p.T;
+  constexpr int PER = (D + 63) / 64, U = 8;
+  float M = -1.0e30f, L = 0.0f, acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.0f;
-  for (int c = 0; c < p.n_chunks; ++c) {
-    const int64_t base = ((int64_t)c * p.BH + bh) * p.T + row;
-    const float w = fast_exp2(p.part_ml[2 * base] - M);
-    L += w * p.part_ml[2 * base + 1];
-    const float* po = p.part_o + base * D;
+  for (int c0 = 0; c0 < p.n_chunks; c0 += 64) {
+    const bool ok = c0 + lane < p.n_chunks && !chunk_unused(p, c0 + lane, q, q);
+    const uint64_t used = __builtin_amdgcn_ballot_w64(ok);
+    if (!used) continue;
+    const float2 ml = ok ? *reinterpret_cast<const float2*>(p.part_ml + 2 * (base0 + (c0 + lane) * bstep))
+                         : float2{-1.0e30f, 0.0f};
+    float mx = ml.x;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int d = lane + 64 * i;
-      if (d < D) acc[i] += w * po[d];
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    const float mn = fmaxf(M, mx), a = fast_exp2(M - mn);
+    M = mn;
+    const float w = ok ? fast_exp2(ml.x - M) : 0.0f;  // this lane's chunk
+    L = L * a + w * ml.y;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) acc[i] *= a;
+    const int cb = __builtin_ctzll(used), ce = 64 - __builtin_clzll(used);
+    for (int c = cb; c < ce; c += U) {
+      float v[U][PER];
+      bool live[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        live[u] = c + u < ce && ((used >> ((c + u) & 63)) & 1);
+        const float* po = p.part_o + (base0 + (int64_t)(c0 + (live[u] ? c + u : cb)) * bstep) * D;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) v[u][i] = lane + 64 * i < D ? po[lane + 64 * i] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float wc = live[u] ? __shfl(w, (c + u) & 63) : 0.0f;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) acc[i] += wc * v[u][i];
+      }
     }
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) L += __shfl_xor(L, off);
   float inv = 1.0f / fmaxf(L, 1.0e-20f);
   if (p.key_mask && !p.key_mask[(int64_t)(bh / p.H) * p.smb + row + p.offset]) inv = 0.0f;
   uint16_t* orow = p.out + (int64_t)bh * p.so0 + row * p.so1;

@@ -518,6 +518,7 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   // split mode (exact tail: no routes): only the tiles of key chunk `chunk`, [c0, c1)
   int64_t c0 = 0, c1 = w1 > f1 ? w1 : f1;
   if (p.n_chunks > 1) {
+    if (chunk_unused(p, chunk, qlo, qhi)) return;  // the merge skips it
     c0 = (int64_t)chunk * p.key_chunk / kTileKeys;
     const int64_t ce = ((int64_t)chunk + 1) * p.key_chunk / kTileKeys;
     if (ce < c1) c1 = ce;

@@ -69,6 +69,13 @@ struct WaveState {
 
 BB_DEV int clamp64(int64_t x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : (int)x); }
 
+// Whether key chunk `chunk` (split mode) holds no key for query positions qlo..qhi: it starts past the last of them,
+// or lies between the front and the first one's window.
+BB_DEV bool chunk_unused(const FlashParams& p, int chunk, int64_t qlo, int64_t qhi) {
+  const int64_t c0 = (int64_t)chunk * p.key_chunk;
+  return c0 > qhi || (c0 >= p.front && c0 + p.key_chunk <= qlo - p.window + 1);
+}
+
 // Window/front mask of one tile for one query row, reduced to int32 thresholds on the tile-relative key kk:
 // valid iff kk <= causal && kk < in_n && (kk < front || kk > win).
 struct WindowMask {
