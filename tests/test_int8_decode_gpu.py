@@ -86,6 +86,21 @@ def test_decode_int8_matches_oracle(n, H, Hkv, d, f16, dev):
     _check(out, ref, f"decode_int8 n={n}")
 
 
+@pytest.mark.parametrize("n,H,Hkv,d", [(16384, 32, 8, 64), (16384, 16, 8, 64), (8192, 16, 8, 128)])
+def test_decode_int8_full_allocation(n, H, Hkv, d, dev):
+    """A cache without spare capacity whose tensors fill their allocations (8 MiB each): no lane may read past the
+    last row. (At head_dim 64 the VALU decode once read 16 bytes per lane where a lane's share is 8.)"""
+    print(f"case decode_int8_full_allocation n={n} H={H}/{Hkv} d={d}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(n)
+    q = torch.randn(H, d, device=dev, generator=g).to(torch.bfloat16)
+    k8, ks = quantize(torch.randn(n, Hkv, d, device=dev, generator=g).to(torch.bfloat16))
+    v8, vs = quantize(torch.randn(n, Hkv, d, device=dev, generator=g).to(torch.bfloat16))
+    assert k8.numel() == 8 << 20
+    out = decode_int8(q, k8, ks, v8, vs, n, d ** -0.5)
+    torch.cuda.synchronize()
+    _check(out, oracle.decode(q, k8, ks, v8, vs, n, d ** -0.5), f"decode_int8_full_allocation n={n}")
+
+
 @pytest.mark.parametrize("n,H,Hkv,d,f16", [(1, 32, 8, 128, True), (2049, 32, 8, 128, False),
                                            (131073, 32, 8, 128, True), (5000, 16, 2, 64, False),
                                            (700, 16, 8, 128, True)])

@@ -179,14 +179,22 @@ __global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeParams p) {
       const int8_t* vr = p.v8 + row * D + DPL * sub;
       ks = load_scale(p.ks, row, p.scale_is_f16);
       vs = load_scale(p.vs, row, p.scale_is_f16);
+      // the lane's DPL bytes and no more: at head_dim 64 a 16-byte load would reach past the last row of the cache
+      uint32_t kw[DPL / 4], vw[DPL / 4];
+      if constexpr (DPL == 16) {
+        const u32x4_t a = ld16(kr), b = ld16(vr);
 #pragma unroll
-      for (int e0 = 0; e0 < DPL; e0 += 16) {
-        const u32x4_t kw = ld16(kr + e0), vw = ld16(vr + e0);
+        for (int i = 0; i < 4; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
+      } else {
+        static_assert(DPL == 8, "8 or 16 bytes per lane");
+        const u32x2_t a = *reinterpret_cast<const u32x2_t*>(kr), b = *reinterpret_cast<const u32x2_t*>(vr);
 #pragma unroll
-        for (int e = 0; e < 16 && e0 + e < DPL; ++e) {
-          kf[e0 + e] = (float)(int8_t)((kw[e >> 2] >> (8 * (e & 3))) & 0xffu);
-          vf[e0 + e] = (float)(int8_t)((vw[e >> 2] >> (8 * (e & 3))) & 0xffu);
-        }
+        for (int i = 0; i < 2; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
+      }
+#pragma unroll
+      for (int e = 0; e < DPL; ++e) {
+        kf[e] = (float)(int8_t)((kw[e >> 2] >> (8 * (e & 3))) & 0xffu);
+        vf[e] = (float)(int8_t)((vw[e >> 2] >> (8 * (e & 3))) & 0xffu);
       }
     } else {
       const uint16_t* kr = p.kb + (int64_t)g * p.skb0 + j * p.skb1 + DPL * sub;
