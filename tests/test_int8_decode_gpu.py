@@ -143,6 +143,41 @@ def test_decode_int8_append_matches_separate_steps(n, H, Hkv, d, f16, dev):
     _check(out, oracle.decode(q, k8, ks, v8, vs, n, d ** -0.5), f"decode_append n={n}")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,H,Hkv,d,layout", [(1, 32, 8, 128, "heads"), (255, 16, 8, 64, "tokens"), (257, 8, 1, 128, "heads"),
+                                              (4099, 32, 8, 128, "tokens"), (20001, 4, 4, 64, "heads"),
+                                              (20001, 16, 2, 64, "tokens"), (300, 8, 8, 128, "odd")])
+def test_one_token_over_16bit_cache(n, H, Hkv, d, layout, dtype, dev):
+    """RDAttention.exact_attention of one token (split-K dense decode) against float64 SDPA: cache views in head-major,
+    token-major and padded-row ("odd", rows not 16-byte aligned: copied; fp16 only) layouts, lengths around one split."""
+    from types import SimpleNamespace
+
+    from bigger_bird_amd import RDAttention
+
+    print(f"case one_token n={n} H={H}/{Hkv} d={d} {layout} {dtype}", flush=True)
+    if layout == "odd" and dtype == torch.bfloat16:
+        layout = "heads"  # decode_bf16 takes 16-byte aligned cache rows only
+    base = SimpleNamespace(config=SimpleNamespace(num_attention_heads=H, num_key_value_heads=Hkv), layer_idx=0, head_dim=d,
+                           scaling=d ** -0.5, q_proj=None, k_proj=None, v_proj=None, o_proj=None)
+    q = _rand((1, H, 1, d), 1).to(dtype)
+    k, v = _rand((1, Hkv, n, d), 2).to(dtype), _rand((1, Hkv, n, d), 3).to(dtype)
+
+    def place(x):
+        if layout == "tokens":
+            return x.to(dev).transpose(1, 2).contiguous().transpose(1, 2)
+        if layout == "odd":
+            buf = torch.zeros(*x.shape[:-1], d + 3, dtype=dtype, device=dev)
+            buf[..., :d] = x.to(dev)
+            return buf[..., :d]
+        return x.to(dev)
+
+    out = RDAttention(base).exact_attention(q.to(dev), place(k), place(v), 1, n)
+    assert out.shape == (1, H, 1, d) and out.dtype == dtype
+    ref = torch.nn.functional.scaled_dot_product_attention(
+        q.double(), k.double().repeat_interleave(H // Hkv, 1), v.double().repeat_interleave(H // Hkv, 1), scale=d ** -0.5)
+    _check(out, ref, f"one_token n={n}")
+
+
 def test_decode_bf16_matches_sdpa(dev):
     print("case decode_bf16", flush=True)
     n, H, Hkv, d = 5000, 32, 8, 128

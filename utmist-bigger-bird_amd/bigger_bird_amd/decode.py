@@ -69,6 +69,25 @@ def bigger_bird_decode(q, k, v, indices, *, front=64, window=4096, scale=1.0, n=
     return out
 
 
+def decode_dense(q, k, v, scale):
+    """One token q [H, D] over every row of a bf16 / fp16 cache k / v [Hkv, N, D] -> [H, D]: bigger_bird_decode with
+    all keys in the window and no routes (fp32 probabilities; split over the chip and merged, two launches)."""
+    h, d = q.shape
+    hk, n, _ = k.shape
+    _lib.require_gpu(q, k, v, what="decode_dense")
+    k, v = _rows16(k), _rows16(v)
+    q = q if q.stride(-1) == 1 else q.contiguous()
+    out = torch.empty(h, d, dtype=q.dtype, device=q.device)
+    L = _lib.lib()
+    ws_bytes = L.bb_sparse_decode_workspace(h, hk, d, hk, 0, n, 0, 0)
+    ws = _lib.workspace(ws_bytes, q.device)
+    _lib.check(L.bb_sparse_decode(
+        _lib.ptr(q), q.stride(0), _lib.ptr(k), _lib.i64s(*k.stride()[:2]), _lib.ptr(v), _lib.i64s(*v.stride()[:2]), None,
+        None, hk, 0, n, None, n, h, hk, d, 0, n, float(scale), 0, int(q.dtype == torch.float16), _lib.ptr(out),
+        out.stride(0), _lib.ptr(ws), ws_bytes, _lib.stream_of(q)))
+    return out
+
+
 def _route(q, k, k_route, front, window, scale, n, splits):
     if not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError("bigger_bird_route requires CUDA FP16/BF16")

@@ -132,11 +132,12 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const int8_t* __restric
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Decode. Workgroup (split s, KV head g): 4 waves; a wave walks keys 8 at a time, 8 lanes per key row (16 d each).
+// INT8 decode on the VALU (the shapes decode_mfma_kernel below is not built for). Workgroup (split s, KV head g): 4
+// waves; a wave walks keys 8 at a time, 8 lanes per key row (D / 8 values each).
 constexpr int kDecThreads = 256;
 constexpr float kDecRescale = 8.0f;
 
-template <int D, int G, bool INT8>
+template <int D, int G>
 __global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeParams p) {
   constexpr int LPK = 8;             // lanes per key
   constexpr int DPL = D / LPK;       // d values per lane
@@ -172,42 +173,26 @@ __global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeParams p) {
 
   for (int64_t j = j_begin + slot; j < j_end; j += SLOTS) {
     float kf[DPL], vf[DPL];
-    float ks = 1.0f, vs = 1.0f;
-    if constexpr (INT8) {
-      const int64_t row = j * p.Hkv + g;
-      const int8_t* kr = p.k8 + row * D + DPL * sub;
-      const int8_t* vr = p.v8 + row * D + DPL * sub;
-      ks = load_scale(p.ks, row, p.scale_is_f16);
-      vs = load_scale(p.vs, row, p.scale_is_f16);
-      // the lane's DPL bytes and no more: at head_dim 64 a 16-byte load would reach past the last row of the cache
-      uint32_t kw[DPL / 4], vw[DPL / 4];
-      if constexpr (DPL == 16) {
-        const u32x4_t a = ld16(kr), b = ld16(vr);
+    const int64_t row = j * p.Hkv + g;
+    const int8_t* kr = p.k8 + row * D + DPL * sub;
+    const int8_t* vr = p.v8 + row * D + DPL * sub;
+    const float ks = load_scale(p.ks, row, p.scale_is_f16), vs = load_scale(p.vs, row, p.scale_is_f16);
+    // the lane's DPL bytes and no more: at head_dim 64 a 16-byte load would reach past the last row of the cache
+    uint32_t kw[DPL / 4], vw[DPL / 4];
+    if constexpr (DPL == 16) {
+      const u32x4_t a = ld16(kr), b = ld16(vr);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
-      } else {
-        static_assert(DPL == 8, "8 or 16 bytes per lane");
-        const u32x2_t a = *reinterpret_cast<const u32x2_t*>(kr), b = *reinterpret_cast<const u32x2_t*>(vr);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
-      }
-#pragma unroll
-      for (int e = 0; e < DPL; ++e) {
-        kf[e] = (float)(int8_t)((kw[e >> 2] >> (8 * (e & 3))) & 0xffu);
-        vf[e] = (float)(int8_t)((vw[e >> 2] >> (8 * (e & 3))) & 0xffu);
-      }
+      for (int i = 0; i < 4; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
     } else {
-      const uint16_t* kr = p.kb + (int64_t)g * p.skb0 + j * p.skb1 + DPL * sub;
-      const uint16_t* vr = p.vb + (int64_t)g * p.svb0 + j * p.svb1 + DPL * sub;
+      static_assert(DPL == 8, "8 or 16 bytes per lane");
+      const u32x2_t a = *reinterpret_cast<const u32x2_t*>(kr), b = *reinterpret_cast<const u32x2_t*>(vr);
 #pragma unroll
-      for (int e0 = 0; e0 < DPL; e0 += 8) {
-        const u32x4_t kw = ld16(kr + e0), vw = ld16(vr + e0);
+      for (int i = 0; i < 2; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
+    }
 #pragma unroll
-        for (int e = 0; e < 8 && e0 + e < DPL; ++e) {
-          kf[e0 + e] = bf16_to_f32((uint16_t)(kw[e >> 1] >> (16 * (e & 1))));
-          vf[e0 + e] = bf16_to_f32((uint16_t)(vw[e >> 1] >> (16 * (e & 1))));
-        }
-      }
+    for (int e = 0; e < DPL; ++e) {
+      kf[e] = (float)(int8_t)((kw[e >> 2] >> (8 * (e & 3))) & 0xffu);
+      vf[e] = (float)(int8_t)((vw[e >> 2] >> (8 * (e & 3))) & 0xffu);
     }
     float s[G];
 #pragma unroll
@@ -586,10 +571,9 @@ hipError_t launch_decode_dg(const DecodeParams& p, hipStream_t stream) {
       hipLaunchKernelGGL(decode_mfma_kernel<true>, dim3(p.n_splits, p.Hkv), dim3(64 * kMdWaves), 0, stream, p);
     else
       hipLaunchKernelGGL(decode_mfma_kernel<false>, dim3(p.n_splits, p.Hkv), dim3(64 * kMdWaves), 0, stream, p);
-  } else if (p.k8)
-    hipLaunchKernelGGL((decode_kernel<D, G, true>), dim3(p.n_splits, p.Hkv), dim3(kDecThreads), 0, stream, p);
-  else
-    hipLaunchKernelGGL((decode_kernel<D, G, false>), dim3(p.n_splits, p.Hkv), dim3(kDecThreads), 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((decode_kernel<D, G>), dim3(p.n_splits, p.Hkv), dim3(kDecThreads), 0, stream, p);
+  }
   hipLaunchKernelGGL(decode_merge_kernel<D>, dim3(p.H, D / kMergeCols), dim3(kMergeThreads), 0, stream, p);
   return hipGetLastError();
 }
@@ -717,6 +701,21 @@ bool decode_fuses_append(const DecodeParams& p) {
 hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
   if (p.n <= 0) return hipErrorInvalidValue;
   if (p.knew != nullptr && !decode_fuses_append(p)) return hipErrorInvalidValue;
+  if (!p.k8) {
+    // A bf16 cache runs on the split-K sparse decode kernel with every key in its window: rows streamed with
+    // line-covering non-temporal loads, two keys per slot in flight. Against the one-key-per-step kernel this used to
+    // be (whole calls, us): 131072 keys of 8 KV heads x 4 query heads 97 -> 91, 16 x 2 180 -> 161, 32 x 1 355 -> 309,
+    // 4 x 8 122 -> 99; 16384 keys of 32 x 1 51 -> 48; the same below 4096 keys, where the launches are the time.
+    SparseDecodeParams s = {};
+    s.q = p.q; s.k = p.kb; s.v = p.vb; s.out = p.out; s.part = p.part;
+    s.sq = p.sq; s.sk0 = p.skb0; s.sk1 = p.skb1; s.sv0 = p.svb0; s.sv1 = p.svb1; s.so = p.so;
+    s.n = s.cap = p.n;
+    s.split_len = p.split_len; s.n_splits = p.n_splits;
+    s.H = p.H; s.Hkv = p.Hkv; s.G = p.H / p.Hkv; s.D = p.D; s.rows = p.Hkv;
+    s.window = p.n;
+    s.c = p.c;
+    return launch_sparse_decode(s, stream);
+  }
   switch (p.D) {
     case 64: return launch_decode_d<64>(p, stream);
     case 128: return launch_decode_d<128>(p, stream);

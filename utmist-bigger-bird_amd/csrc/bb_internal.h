@@ -127,8 +127,8 @@ struct SparseDecodeParams {
   uint16_t* out;         // [H, D] (row stride so)
   float* part;           // [H][n_splits][D + 2]
   int64_t sq, sk0, sk1, sv0, sv1, si0, si1, so;
-  int64_t n, cap, split_len;
-  int H, Hkv, G, D, rows, front, window, route_k, n_splits, f16;
+  int64_t n, cap, split_len, window;
+  int H, Hkv, G, D, rows, front, route_k, n_splits, f16;
   float c;               // scale * log2(e)
   RowAppend app;         // the step's new row (dense decode without routing), or app.knew = null
   int64_t* n_advance;    // after the merge: *n_advance += advance when the row was appended (n_advance = n_dev), or null
