@@ -103,6 +103,33 @@ def test_tail_window_n_is_dense_causal_rows(dtype, heads, dev):
     _check(out, ref, "tail_split")
 
 
+@pytest.mark.parametrize("H,Hkv,T,N,front,window,rk,groups", [
+    (8, 2, 700, 700, 64, 128, 64, 1), (8, 4, 1501, 1501, 16, 256, 130, 1), (4, 4, 1100, 1400, 7, 97, 33, 1),
+    (8, 2, 2300, 2300, 64, 512, 600, 1),   # past one 512-slot pass of the route list
+    (16, 2, 1200, 1200, 64, 128, 64, 5),   # several route groups: batches gathered in the kernel
+    (8, 2, 64, 64, 0, 64, 0, 1), (8, 2, 65, 129, 64, 1, 8, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_d64_pipelined(H, Hkv, T, N, front, window, rk, groups, dtype, dev):
+    """head_dim 64 on the pipelined kernel (4, 2 and 1 query heads per workgroup) against the float64 oracle."""
+    print(f"case d64_pipelined {H}/{Hkv} T={T} N={N} front={front} window={window} rk={rk} groups={groups} {dtype}", flush=True)
+    d, g = 64, torch.Generator().manual_seed(T + rk)
+    q, k, v = _rand((H, T, d), 51, dtype), _rand((Hkv, N, d), 52, dtype), _rand((Hkv, N, d), 53, dtype)
+    chunk = 256 if groups > 1 else None
+    span = max(N - window - front, 1)
+    idx = torch.full((H, groups, rk), -1, dtype=torch.int32)
+    for h in range(H):
+        for gi in range(groups):
+            m = min(rk - h % 3, span) if rk else 0
+            idx[h, gi, :max(m, 0)] = (torch.randperm(span, generator=g)[:max(m, 0)] + front).to(torch.int32)
+    out = bigger_bird_flash(q.to(dev), k.to(dev), v.to(dev), idx.to(dev), front=front, window=window, num_heads=H,
+                            kv_groups=H // Hkv, scale=d ** -0.5, route_chunk=chunk)
+    rows = torch.stack(torch.meshgrid(torch.arange(H), torch.arange(T), indexing="ij"), -1).reshape(-1, 2)
+    rows = rows[torch.randperm(rows.shape[0], generator=g)[:6000]]
+    ref = oracle.attn_rows(q, k, v, idx, rows, front=front, window=window, num_heads=H, kv_groups=H // Hkv,
+                           scale=d ** -0.5, route_chunk=chunk)
+    _check(out[rows[:, 0], rows[:, 1]], ref, "d64_pipelined")
+
+
 @pytest.mark.parametrize("t,n,front,window,noncausal", [
     (2, 257, 0, 257, True), (65, 1023, 0, 1023, True), (1, 4099, 0, 4099, True),  # a handful of tiles; one row
     (300, 700, 0, 700, False), (130, 2049, 0, 2049, False),  # causal rows that end inside and before later chunks

@@ -150,13 +150,12 @@ int64_t bb_transpose_v_cols(int64_t N) { return cdiv(N > 0 ? N : 1, 64) * 64; }
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Routed tiles are pre-gathered for the pipelined kernel (head_dim 128, query heads per KV head a multiple of 4, no
-// token mask) when the route list has a single group. With several groups (vertical_scope) most groups are empty and
+// Routed tiles are pre-gathered for the pipelined kernel (head_dim 64 or 128, no token mask) when the route list has a single group. With several groups (vertical_scope) most groups are empty and
 // the tiles of every group would cost BH x groups x 32 KB per 64 slots, so the kernel gathers the batches it uses
 // itself. K rows of 4 GiB or more per KV head also leave the pipelined kernel; the reservation does not see the row
 // stride and is made anyway (it is small next to such K).
 static bool routed_tiles_wanted(int D, int kv_groups, int route_k, int n_groups, bool key_mask) {
-  return route_k > 0 && n_groups == 1 && !key_mask && D == 128 && kv_groups > 0 && flash_pipe_enabled();
+  return route_k > 0 && n_groups == 1 && !key_mask && (D == 64 || D == 128) && kv_groups > 0 && flash_pipe_enabled();
 }
 
 size_t bb_sparse_flash_workspace(int BH, int64_t T, int64_t N, int D, int num_heads, int kv_groups, int64_t front,
@@ -169,7 +168,7 @@ size_t bb_sparse_flash_workspace(int BH, int64_t T, int64_t N, int D, int num_he
   size_t bytes = 0;
   if (!have_vt) bytes += align256((size_t)(BH / kv_groups) * D * bb_transpose_v_cols(N) * 2);
   if (routed_tiles_wanted(D, kv_groups, route_k, n_groups, has_key_mask != 0))
-    bytes += align256(bb::route_tiles_bytes(BH, n_groups, route_k));
+    bytes += align256(bb::route_tiles_bytes(BH, n_groups, route_k, D));
   if (s.split) bytes += (size_t)s.n_chunks * BH * T * (size_t)(D + 2) * sizeof(float);
   return bytes;
 }
@@ -270,22 +269,22 @@ static int sparse_flash_impl(const void* q, const int64_t* sq, const void* k, co
   const bool pipe = flash_pipe_enabled() && bb::flash_pipe_supported(p, D, s.hpw);
   if (routed_tiles_wanted(D, kv_groups, route_k, p.n_groups, key_mask != nullptr)) {
     uint16_t* rt = reinterpret_cast<uint16_t*>(wsp);
-    wsp += align256(bb::route_tiles_bytes(BH, p.n_groups, route_k));
+    wsp += align256(bb::route_tiles_bytes(BH, p.n_groups, route_k, D));
     if (pipe) {
       p.rtiles = rt;
       p.rt_batches = (int)cdiv(route_k, 64);
-      hipError_t e = bb::launch_route_tiles(p, rt, st);
+      hipError_t e = bb::launch_route_tiles(p, D, rt, st);
       if (e != hipSuccess) return hip_status(e, "bb_sparse_flash routed tiles");
     }
   }
   if (s.split) {
     p.part_o = reinterpret_cast<float*>(wsp);
     p.part_ml = p.part_o + (size_t)s.n_chunks * BH * T * D;
-    hipError_t e = pipe ? bb::launch_flash_pipe(p, s.hpw, st) : bb::launch_flash(p, D, s.hpw, true, st);
+    hipError_t e = pipe ? bb::launch_flash_pipe(p, D, s.hpw, st) : bb::launch_flash(p, D, s.hpw, true, st);
     if (e != hipSuccess) return hip_status(e, "bb_sparse_flash split kernel");
     return hip_status(bb::launch_flash_merge(p, D, st), "bb_sparse_flash merge kernel");
   }
-  if (pipe) return hip_status(bb::launch_flash_pipe(p, s.hpw, st), "bb_sparse_flash pipelined kernel");
+  if (pipe) return hip_status(bb::launch_flash_pipe(p, D, s.hpw, st), "bb_sparse_flash pipelined kernel");
   return hip_status(bb::launch_flash(p, D, s.hpw, false, st), "bb_sparse_flash kernel");
 }
 

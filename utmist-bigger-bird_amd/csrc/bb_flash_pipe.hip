@@ -1,5 +1,5 @@
-// Ping-pong sink + causal window + routed sparse flash attention for gfx950 (head_dim 128, no token mask): the main
-// pass of Bigger Bird v3 prefill at production shape.
+// Ping-pong sink + causal window + routed sparse flash attention for gfx950 (head_dim 128 or 64, no token mask): the
+// main pass of Bigger Bird v3 prefill.
 //
 // Same semantics as bb_flash.hip (kernels/bigger_bird_flash.py:42-96 of the reference). Work decomposition:
 //   * a workgroup = 8 waves = the 4 query heads of one KV head x 2 blocks of 32 query rows (64 rows); every K / V^T
@@ -19,6 +19,12 @@
 //     resource bounds;
 //   * the exponent offset moves only when a probability would exceed 2^8 (O rescales stay rare); tiles without masked
 //     elements skip the per-tile maximum unless the row sum says the offset must move;
+//   * head_dim 64 runs the same structure with half the MFMAs and LDS bytes per tile (64 KB of LDS), so the softmax of
+//     a tile, not its MFMAs, is the longer phase. What bounds it is the SIMD's issue: a wave's 32 x 64 softmax takes
+//     312 ns alone and 461 ns beside another wave's 32 MFMAs (measured on the bare instruction streams), the loop
+//     about 515 ns per tile. 20011 tokens, window 4096, 512 routed keys, 32 heads over 8: 1146 us on the kernel
+//     without phases (bb_flash.hip), 743 us here; two tiles per phase pair measured the same (773-792 against
+//     780-788 us before the loads moved to the MFMA phase);
 //   * routed keys differ per head: after the window loop the waves of a head stream its routed K / V^T tiles into
 //     that head's LDS tile, pre-gathered per 64-slot batch by route_tiles_kernel (one route group), or gather the
 //     batch's K rows and V rows themselves (several route groups: the GATHER instantiation).
@@ -43,24 +49,38 @@
 namespace bb {
 namespace {
 
-constexpr int PD = 128;                 // head_dim
 constexpr int PNW = 8;                  // waves per workgroup
 constexpr int PHEADS = 4;               // most query heads per workgroup (HPW = 4, 2 or 1 share each tile)
-constexpr int PTE = kTileKeys * PD;     // elements of one K (or V^T) tile
 constexpr int PST = 4;                  // ring stages, each a K tile and a V^T tile
-constexpr int PBLK = PTE * 2 / 1024;    // 1 KB direct-load blocks per tile (16)
-constexpr int PLDS = PST * 2 * PTE;     // 128 KB; the routed phase reuses it as 4 heads x (K + V^T)
 constexpr int kRouteCache = 512;        // route slots per head staged in LDS at a time
-static_assert(PHEADS * 2 * PTE <= PLDS, "routed tiles fit the ring");
+static_assert(PHEADS <= PST, "routed tiles (4 heads x (K + V^T)) fit the ring");
+
+template <int D>
+struct Pipe {
+  static_assert(D == 64 || D == 128, "head_dim 64 or 128");
+  static constexpr int TE = kTileKeys * D;      // elements of one K (or V^T) tile
+  static constexpr int BLK = TE * 2 / 1024;     // 1 KB direct-load blocks per tile
+  static constexpr int LOADS = 2 * BLK / PNW;   // direct loads per wave and tile (K and V^T)
+  static constexpr int LDS = PST * 2 * TE;      // 128 KB (64 KB at D = 64)
+  static constexpr int LPR = D / 8;             // 16-byte chunks per K row
+  static constexpr int NV = D / 8, NK = D / 8;  // V^T and K fragments of an MFMA phase
+};
 
 typedef __attribute__((__vector_size__(4 * sizeof(int32_t)))) int32_t i32x4_t;
 
 // LDS tile layouts of this kernel.
-// K tile: key row r (0..63), 16-byte chunk c (d = 8c..8c+7) at element r * PD + 8 (c ^ pk_swz(r)). The 16 keys an MFMA
+// K tile: key row r (0..63), 16-byte chunk c (d = 8c..8c+7) at element r * D + 8 (c ^ pk_swz(r)). The 16 keys an MFMA
 // key block reads at one d chunk ({0-7, 16-23} + 8 (kb % 2) + 32 (kb / 2)) sit in 16 distinct slots, and pk_swz does
 // not change when a row moves by 8 (within those sets) or by 32, so a lane's fragment offsets are fixed per d chunk.
-BB_DEV int pk_swz(int r) { return (r & 7) | ((r >> 1) & 8); }
-BB_DEV int pk_off(int r, int c) { return r * PD + 8 * (c ^ pk_swz(r)); }
+// At D = 64 a row is half of the 16 bank slots, so rows of one parity share a half and the swizzle has 3 bits: in each
+// of the four 16-lane groups that serve a fragment read (below) the 8 rows of a parity get 8 slots.
+template <int D>
+BB_DEV int pk_swz(int r) {
+  if constexpr (D == 64) return ((r >> 1) & 3) | ((((r >> 2) ^ (r >> 4)) & 1) << 2);
+  else return (r & 7) | ((r >> 1) & 8);
+}
+template <int D>
+BB_DEV int pk_off(int r, int c) { return r * D + 8 * (c ^ pk_swz<D>(r)); }
 // V^T tile: row d (0..127), 8-key unit u of the global V^T layout at element d * 64 + 8 ((u + pv_rot(d)) & 7). The
 // rotation depends on d % 16 only, so the d block of a fragment is an immediate offset. A ds_read_b128 serves its 64
 // lanes in four 16-lane groups (measured on gfx950: lanes 32 h + 4 q + 0..3 for the quads q whose three index bits
@@ -129,7 +149,9 @@ struct PipeWindowMask {  // front | causal window (nothing when !any)
 // Direct global->LDS tile loads through buffer resources (one per KV head: rows past N read as zeros, and every
 // per-lane offset is a loop-invariant 32-bit value). Block b (1 KB) of a tile is loaded by wave b % 8; its lanes
 // land at byte 16 * lane of the block.
+template <int D>
 struct TileLoader {
+  using P = Pipe<D>;
   __amdgpu_buffer_rsrc_t krs, vrs;
   uint32_t kvoff, vvoff;    // per-lane byte offsets of this wave's first block
   uint32_t kstep, vstep;    // byte distance between this wave's two blocks (8 blocks apart)
@@ -142,11 +164,11 @@ struct TileLoader {
     krow_bytes = (uint32_t)(sk1 * 2);
     // num_records is an unsigned 32-bit byte count (passed through int): sizes up to 4 GiB
     krs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), 0, (int)(uint32_t)(N * sk1 * 2), 0x00020000);
-    vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vtbase), 0, (int)(uint32_t)(PD * np * 2), 0x00020000);
-    // K block b = w + 8i: row 4b + lane/16, LDS slot lane%16 holds chunk (lane%16) ^ pk_swz(row); pk_swz(row) does
-    // not depend on i (rows 32 apart)
-    const int krow = 4 * w + lane / 16;
-    kvoff = (uint32_t)krow * krow_bytes + 16u * (uint32_t)((lane % 16) ^ pk_swz(krow));
+    vrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(vtbase), 0, (int)(uint32_t)(D * np * 2), 0x00020000);
+    // K block b = w + 8i: LPR lanes per row, row (64 / LPR) b + lane / LPR, LDS slot lane % LPR holds chunk
+    // (lane % LPR) ^ pk_swz(row); pk_swz(row) does not depend on i (rows 32 apart at D = 128, one block at D = 64)
+    const int krow = 64 / P::LPR * w + lane / P::LPR;
+    kvoff = (uint32_t)krow * krow_bytes + 16u * (uint32_t)((lane % P::LPR) ^ pk_swz<D>(krow));
     kstep = 32u * krow_bytes;
     // V^T block b = w + 8i: d = 8b + lane/8, LDS slot lane%8 holds unit (lane%8 - pv_rot(d)) & 7; pv_rot(d) does
     // not depend on i (rows 64 apart)
@@ -159,13 +181,13 @@ struct TileLoader {
     // offset), so rows past N read as zeros instead of touching memory past the tensor.
     const uint32_t kb = kvoff + (uint32_t)k0 * krow_bytes, vb = (uint32_t)k0 * 2u;
 #pragma unroll
-    for (int i = 0; i < PBLK / PNW; ++i)
+    for (int i = 0; i < P::BLK / PNW; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           krs, reinterpret_cast<__attribute__((address_space(3))) void*>(
                    reinterpret_cast<uintptr_t>(kl + (wave + PNW * i) * 512)),
           16, kb + i * kstep, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < PBLK / PNW; ++i)
+    for (int i = 0; i < P::BLK / PNW; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           vrs, reinterpret_cast<__attribute__((address_space(3))) void*>(
                    reinterpret_cast<uintptr_t>(vt + (wave + PNW * i) * 512)),
@@ -173,9 +195,10 @@ struct TileLoader {
   }
 };
 
+template <int D>
 BB_DEV void vm_wait_tile(bool one_tile_in_flight) {
-  // vmcnt(4) keeps the most recent tile's 4 loads (2 K + 2 V^T blocks) in flight; vmcnt(0) drains everything
-  if (one_tile_in_flight) __builtin_amdgcn_s_waitcnt(0x0F74);
+  // vmcnt(LOADS) keeps the most recent tile's loads in flight; vmcnt(0) drains everything
+  if (one_tile_in_flight) __builtin_amdgcn_s_waitcnt(0x0F70 | Pipe<D>::LOADS);
   else __builtin_amdgcn_s_waitcnt(0x0F70);
 }
 
@@ -191,26 +214,29 @@ BB_DEV void ring_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
+template <int D>
 struct PingState {
-  bf16x8_t qf[2][PD / 32];  // Q^T fragments: row block rb, d step ds (32 d each)
-  f32x4_t o[PD / 16][2];    // O^T: d block db (16 d), row block rb
+  bf16x8_t qf[2][D / 32];   // Q^T fragments: row block rb, d step ds (32 d each)
+  f32x4_t o[D / 16][2];     // O^T: d block db (16 d), row block rb
   f32x4_t s[4][2];          // S^T of the current tile: key block kb (16 keys), row block rb
   bf16x8_t pk[2][2];        // P^T fragments of the previous tile: 32-key step st, row block rb
   float m[2], l[2];         // per row block: exponent offset (log2 units), this lane's share of the row sum
 };
 
-// Per-lane byte offsets of the fragments inside a K tile (k[ds]: key block 0; block kb is 256 (32 (kb / 2) +
+// Per-lane byte offsets of the fragments inside a K tile (k[ds]: key block 0; block kb is 2 D (32 (kb / 2) +
 // 8 (kb % 2)) bytes on) and a V^T tile (v[st]: d block 0; d block db is 2048 db bytes on). With them a fragment
 // address is one add of the tile's wave-uniform LDS address plus an immediate.
+template <int D>
 struct FragOfs {
-  uint32_t k[PD / 32];
+  uint32_t k[D / 32];
   uint32_t v[2];
 };
-BB_DEV FragOfs frag_ofs(int x, int a) {
-  FragOfs f;
+template <int D>
+BB_DEV FragOfs<D> frag_ofs(int x, int a) {
+  FragOfs<D> f;
   const int r0 = 16 * (x >> 3) + (x & 7);  // key row of M-row x in key block 0
 #pragma unroll
-  for (int ds = 0; ds < PD / 32; ++ds) f.k[ds] = 2u * (uint32_t)pk_off(r0, 4 * ds + a);
+  for (int ds = 0; ds < D / 32; ++ds) f.k[ds] = 2u * (uint32_t)pk_off<D>(r0, 4 * ds + a);
 #pragma unroll
   for (int st = 0; st < 2; ++st) f.v[st] = 2u * (uint32_t)pv_off(x, 4 * st + a);
   return f;
@@ -224,14 +250,16 @@ BB_DEV u32x4_t lds16(uint32_t addr) {
 }
 // The tile's fragment base addresses, one add each, kept opaque so that the per-fragment constants go into the
 // ds_read offset field instead of being folded into the scalar and added per read.
+template <int D>
 struct FragBase {
-  uint32_t k[PD / 32];
+  uint32_t k[D / 32];
   uint32_t v[2];
 };
-BB_DEV FragBase frag_base(uint32_t kl, uint32_t vt, const FragOfs& f) {
-  FragBase b;
+template <int D>
+BB_DEV FragBase<D> frag_base(uint32_t kl, uint32_t vt, const FragOfs<D>& f) {
+  FragBase<D> b;
 #pragma unroll
-  for (int j = 0; j < PD / 32; ++j) {
+  for (int j = 0; j < D / 32; ++j) {
     b.k[j] = kl + f.k[j];
     asm volatile("" : "+v"(b.k[j]));
   }
@@ -242,76 +270,79 @@ BB_DEV FragBase frag_base(uint32_t kl, uint32_t vt, const FragOfs& f) {
   }
   return b;
 }
-// Fragment i of an MFMA phase: i < 16 the V^T fragment of PV step (st, db) = (i / 8, i % 8); 16 + j the K fragment of
-// QK step (kb, ds) = (j % 4, j / 4) (consecutive K fragments belong to different key blocks, so each accumulator's
-// chain over ds has three other blocks' MFMAs between its steps).
-BB_DEV u32x4_t ping_frag_at(const FragBase& b, int i) {
-  if (i < 16) return lds16(b.v[i / 8] + 2048u * (uint32_t)(i % 8));
-  const int j = i - 16, kb = j % 4, ds = j / 4;
-  return lds16(b.k[ds] + 256u * (uint32_t)(32 * (kb >> 1) + 8 * (kb & 1)));
+// Fragment i of an MFMA phase: i < NV the V^T fragment of PV step (st, db) = (i / (D / 16), i % (D / 16)); NV + j the
+// K fragment of QK step (kb, ds) = (j % 4, j / 4) (consecutive K fragments belong to different key blocks, so each
+// accumulator's chain over ds has three other blocks' MFMAs between its steps).
+template <int D>
+BB_DEV u32x4_t ping_frag_at(const FragBase<D>& b, int i) {
+  if (i < Pipe<D>::NV) return lds16(b.v[i / (D / 16)] + 2048u * (uint32_t)(i % (D / 16)));
+  const int j = i - Pipe<D>::NV, kb = j % 4, ds = j / 4;
+  return lds16(b.k[ds] + 2u * D * (uint32_t)(32 * (kb >> 1) + 8 * (kb & 1)));
 }
 
-template <bool F16>
-BB_DEV void ping_mma(PingState& st, int i, bf16x8_t a) {
-  if (i < 16) {
-    const int stp = i / 8, db = i % 8;
+template <bool F16, int D>
+BB_DEV void ping_mma(PingState<D>& st, int i, bf16x8_t a) {
+  if (i < Pipe<D>::NV) {
+    const int stp = i / (D / 16), db = i % (D / 16);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) st.o[db][rb] = mma16<F16>(a, st.pk[stp][rb], st.o[db][rb]);
   } else {
-    const int j = i - 16, kb = j % 4, ds = j / 4;
+    const int j = i - Pipe<D>::NV, kb = j % 4, ds = j / 4;
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) st.s[kb][rb] = mma16<F16>(a, st.qf[rb][ds], st.s[kb][rb]);
   }
 }
 
-BB_DEV void clear_s(PingState& st) {
+template <int D>
+BB_DEV void clear_s(PingState<D>& st) {
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) st.s[kb][rb] = zero4();
 }
 
-// S(t) = K Q^T (32 MFMAs on 16 K fragments).
-template <bool F16>
-BB_DEV void ping_qk(PingState& st, const uint16_t* kl, const FragOfs& fo) {
-  const FragBase fb = frag_base(lds_addr(kl), 0u, fo);
+// S(t) = K Q^T (32 MFMAs on 16 K fragments at D = 128, half of that at 64).
+template <bool F16, int D>
+BB_DEV void ping_qk(PingState<D>& st, const uint16_t* kl, const FragOfs<D>& fo) {
+  const FragBase<D> fb = frag_base(lds_addr(kl), 0u, fo);
   clear_s(st);
 #pragma unroll
-  for (int i = 16; i < 32; ++i) ping_mma<F16>(st, i, as_bf16x8(ping_frag_at(fb, i)));
+  for (int i = Pipe<D>::NV; i < Pipe<D>::NV + Pipe<D>::NK; ++i) ping_mma<F16>(st, i, as_bf16x8(ping_frag_at(fb, i)));
 }
 
-// O^T += V^T P^T (32 MFMAs on 16 V^T fragments).
-template <bool F16>
-BB_DEV void ping_pv(PingState& st, const uint16_t* vt, const FragOfs& fo) {
-  const FragBase fb = frag_base(0u, lds_addr(vt), fo);
+// O^T += V^T P^T (32 MFMAs on 16 V^T fragments at D = 128).
+template <bool F16, int D>
+BB_DEV void ping_pv(PingState<D>& st, const uint16_t* vt, const FragOfs<D>& fo) {
+  const FragBase<D> fb = frag_base(0u, lds_addr(vt), fo);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) ping_mma<F16>(st, i, as_bf16x8(ping_frag_at(fb, i)));
+  for (int i = 0; i < Pipe<D>::NV; ++i) ping_mma<F16>(st, i, as_bf16x8(ping_frag_at(fb, i)));
 }
 
-// MFMA phase of the window loop: O^T += V^T(t-1) P(t-1)^T, then S(t) = K(t) Q^T (64 MFMAs), with the 32 LDS fragment
-// reads software-pipelined six fragments ahead through a register ring (the LDS latency would otherwise idle the
-// matrix core between each read and the MFMAs that consume it; 4 and 8 ahead measured slower).
+// MFMA phase of the window loop: O^T += V^T(t-1) P(t-1)^T, then S(t) = K(t) Q^T (64 MFMAs at D = 128), with the 32 LDS
+// fragment reads software-pipelined six fragments ahead through a register ring (the LDS latency would otherwise idle
+// the matrix core between each read and the MFMAs that consume it; 4 and 8 ahead measured slower).
 constexpr int kRing = 6;
 
-template <bool F16>
-BB_DEV void ping_mfma_phase(PingState& st, uint32_t kl, uint32_t vt, const FragOfs& fo) {
-  const FragBase fb = frag_base(kl, vt, fo);
+template <bool F16, int D>
+BB_DEV void ping_mfma_phase(PingState<D>& st, uint32_t kl, uint32_t vt, const FragOfs<D>& fo) {
+  constexpr int NF = Pipe<D>::NV + Pipe<D>::NK;
+  const FragBase<D> fb = frag_base(kl, vt, fo);
   u32x4_t ring[kRing];
 #pragma unroll
   for (int i = 0; i < kRing; ++i) ring[i] = ping_frag_at(fb, i);
   clear_s(st);
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
+  for (int i = 0; i < NF; ++i) {
     const bf16x8_t a = as_bf16x8(ring[i % kRing]);
     ping_mma<F16>(st, i, a);
-    if (i + kRing < 32) ring[i % kRing] = ping_frag_at(fb, i + kRing);
+    if (i + kRing < NF) ring[i % kRing] = ping_frag_at(fb, i + kRing);
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 // P(t) = 2^(S(t) c - m) as 16-bit MFMA fragments; sum[rb] = this lane's sum of row block rb's fp32 values.
-template <bool F16>
-BB_DEV void ping_exp(PingState& st, float c, float (&sum)[2]) {
+template <bool F16, int D>
+BB_DEV void ping_exp(PingState<D>& st, float c, float (&sum)[2]) {
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const float nm = -st.m[rb];
@@ -330,7 +361,8 @@ BB_DEV void ping_exp(PingState& st, float c, float (&sum)[2]) {
 }
 
 // Tile maximum of S(t) over the 64 keys of row block rb's row, times c.
-BB_DEV float ping_tile_max(const PingState& st, int rb, float c) {
+template <int D>
+BB_DEV float ping_tile_max(const PingState<D>& st, int rb, float c) {
   // NaN-propagating maximum (v_maximum3_f32): fmaxf would first canonicalise every MFMA result
   float mx = __builtin_elementwise_maximum(st.s[0][rb][0], st.s[1][rb][0]);
 #pragma unroll
@@ -342,12 +374,13 @@ BB_DEV float ping_tile_max(const PingState& st, int rb, float c) {
 }
 
 // Moves the exponent offset of row block rb to mt where `need`, rescaling its O and l.
-BB_DEV void ping_rescale(PingState& st, int rb, bool need, float mt) {
+template <int D>
+BB_DEV void ping_rescale(PingState<D>& st, int rb, bool need, float mt) {
   const float alpha = need ? fast_exp2(st.m[rb] - mt) : 1.0f;
   if (need) st.m[rb] = mt;
   st.l[rb] *= alpha;
 #pragma unroll
-  for (int db = 0; db < PD / 16; ++db)
+  for (int db = 0; db < D / 16; ++db)
 #pragma unroll
     for (int i = 0; i < 4; ++i) st.o[db][rb][i] *= alpha;
 }
@@ -355,8 +388,8 @@ BB_DEV void ping_rescale(PingState& st, int rb, bool need, float mt) {
 // Online softmax of a masked tile S(t) into P(t): running offset m (log2 units), sum l, O rescaled when the tile
 // maximum exceeds m by more than kRescaleThreshold. bits(rb, kb) gives the 4 valid-key bits of key block kb for row
 // block rb's row.
-template <bool F16, typename Bits>
-BB_DEV void ping_softmax_masked(PingState& st, float c, const Bits& bits) {
+template <bool F16, int D, typename Bits>
+BB_DEV void ping_softmax_masked(PingState<D>& st, float c, const Bits& bits) {
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -387,8 +420,8 @@ BB_DEV void ping_softmax_masked(PingState& st, float c, const Bits& bits) {
 // only when a probability may exceed 2^kRescaleThreshold (a lane's partial sum of a row does: every term is at most
 // that sum; an infinite or NaN sum counts too) is the tile maximum taken, the offset moved and the tile exponentiated
 // again. Same bound on P as the masked form, without a maximum per tile in the common case.
-template <bool F16>
-BB_DEV void ping_softmax_open(PingState& st, float c) {
+template <bool F16, int D>
+BB_DEV void ping_softmax_open(PingState<D>& st, float c) {
   float sum[2];
   ping_exp<F16>(st, c, sum);
   const float lim = __builtin_amdgcn_exp2f(kRescaleThreshold);
@@ -450,11 +483,13 @@ BB_DEV PipeItem pipe_item(const FlashParams& p, int bid, int hd, int rbk) {
 // are pre-gathered); a separate instantiation, so that the common kernel's register allocation is not affected.
 // HPW: query heads per workgroup (4 when a KV head serves a multiple of 4 query heads; 2 and 1 for 2 and 1, with
 // 4 and 8 row blocks of 32 rows), so every staged K / V^T tile is read by all 8 waves in each case.
-template <bool F16, bool GATHER, int HPW>
+template <bool F16, bool GATHER, int HPW, int D>
 __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) {
+  constexpr int PTE = Pipe<D>::TE, PBLK = Pipe<D>::BLK;
+  constexpr bool kLoadInMfmaPhase = D == 64;
   static_assert(HPW == 4 || HPW == 2 || HPW == 1, "4, 2 or 1 query heads per workgroup");
   constexpr int RB = PNW / HPW;  // row blocks (waves) per head
-  __shared__ __attribute__((aligned(1024))) uint16_t smem[PLDS];
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[Pipe<D>::LDS];
   __shared__ __attribute__((aligned(16))) int32_t route_keys[HPW][kRouteCache];
   __shared__ int head_batches[RB][HPW];
 
@@ -471,19 +506,19 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   const bool wave_live = it.wave_live;
   const int64_t qw0 = it.qw0, qw1 = it.qw1;
 
-  PingState st;
+  PingState<D> st;
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const int64_t row = rw + 16 * rb + x;
     const bool live = row < T_eff;
     const uint16_t* qrow = p.q + (int64_t)bh * p.sq0 + (live ? row : T_eff - 1) * p.sq1 + 8 * a;
 #pragma unroll
-    for (int ds = 0; ds < PD / 32; ++ds) {
+    for (int ds = 0; ds < D / 32; ++ds) {
       const u32x4_t v = ld16(qrow + 32 * ds);
       st.qf[rb][ds] = as_bf16x8(live ? v : u32x4_t{0, 0, 0, 0});
     }
 #pragma unroll
-    for (int db = 0; db < PD / 16; ++db) st.o[db][rb] = zero4();
+    for (int db = 0; db < D / 16; ++db) st.o[db][rb] = zero4();
     st.m[rb] = -1.0e20f;
     st.l[rb] = 0.0f;
   }
@@ -491,7 +526,7 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   const int64_t qx0 = qw0 + x * p.pos_step, qx1 = qx0 + 16 * p.pos_step;
 
   const uint16_t* kbase = p.k + (int64_t)kvbh * p.sk0;
-  const uint16_t* vtbase = p.vt + (int64_t)kvbh * PD * p.np;
+  const uint16_t* vtbase = p.vt + (int64_t)kvbh * D * p.np;
 
   // ---- tiles (64-aligned): front range [0, f1) and window range [w0, w1) ----
   const int64_t front_end = p.front < qhi + 1 ? p.front : qhi + 1;
@@ -566,20 +601,20 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   uint16_t* ring = smem;
   auto kst = [&](int t) { return ring + (t & (PST - 1)) * 2 * PTE; };
   auto vst = [&](int t) { return ring + (t & (PST - 1)) * 2 * PTE + PTE; };
-  const FragOfs fo = frag_ofs(x, a);
-  TileLoader ld;
+  const FragOfs<D> fo = frag_ofs<D>(x, a);
+  TileLoader<D> ld;
   ld.init(kbase, p.sk1, p.N, vtbase, p.np, wave, lane);
 
   if (ntot > 0) {
     ld.tile(kst(0), vst(0), upos(0));
     if (ntot > 1) ld.tile(kst(1), vst(1), upos(1));
-    vm_wait_tile(ntot > 1);
+    vm_wait_tile<D>(ntot > 1);
     ring_barrier();
     if (grp == 1) ring_barrier();  // waves 4..7 run one phase behind
     // tile 0: QK only
     if (ntot > 2) ld.tile(kst(2), vst(2), upos(2));
     ping_qk<F16>(st, kst(0), fo);
-    vm_wait_tile(ntot > 2);
+    vm_wait_tile<D>(ntot > 2);
     ring_barrier();
     softmax(0);
     ring_barrier();
@@ -589,14 +624,19 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
       // MFMA phase: PV of tile t-1, QK of tile t
       __builtin_amdgcn_s_setprio(1);
       ping_mfma_phase<F16>(st, lds_addr(kst(t)), lds_addr(vst(t - 1)), fo);
+      // Tile t+2 starts loading into the stage tile t-2 used: every wave is past the MFMA phase that last read it (the
+      // other group has at least finished its MFMA phase t-1). Issuing a direct load stalls the wave for as long as
+      // the CU's address unit is busy with the other waves' loads, so the loads go with the shorter phase: at D = 64
+      // the MFMA phase (32 MFMAs against the softmax of the same 64 keys; 780 -> 743 us at 20011 tokens, window 4096,
+      // 32 heads over 8), at D = 128 the VALU phase, after the exponentials.
+      const bool more = t + 2 < ntot;
+      if (kLoadInMfmaPhase && more) ld.tile(kst(t + 2), vst(t + 2), upos(t + 2));
       __builtin_amdgcn_s_setprio(0);
-      vm_wait_tile(false);  // tile t+1 has landed
+      vm_wait_tile<D>(kLoadInMfmaPhase && more);  // tile t+1 has landed
       ring_barrier();
-      // VALU phase: softmax of tile t, then tile t+2 starts loading into the stage tile t-2 used (every wave is past
-      // the MFMA phase that last read it). The loads come after the exponentials: issuing a direct load stalls the
-      // wave for as long as the CU's address unit is busy with the other waves' loads.
+      // VALU phase: softmax of tile t
       ping_softmax_open<F16>(st, p.c);
-      if (t + 2 < ntot) ld.tile(kst(t + 2), vst(t + 2), upos(t + 2));
+      if (!kLoadInMfmaPhase && more) ld.tile(kst(t + 2), vst(t + 2), upos(t + 2));
       ring_barrier();
     }
     // every tile of this loop is masked: t >= max(nu, 1) >= nu
@@ -605,7 +645,7 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
       __builtin_amdgcn_s_setprio(1);
       ping_mfma_phase<F16>(st, lds_addr(kst(t)), lds_addr(vst(t - 1)), fo);
       __builtin_amdgcn_s_setprio(0);
-      vm_wait_tile(false);
+      vm_wait_tile<D>(false);
       ring_barrier();
       softmax_masked(t);
       if (t + 2 < ntot) ld.tile(kst(t + 2), vst(t + 2), upos(t + 2));
@@ -696,12 +736,12 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
             const uint16_t* vb = p.v + (int64_t)it.kvbh * p.sv0;
             for (int b = rbk; b < PBLK; b += RB) {
               const int e = b * 512 + 8 * lane;
-              const int row = e / PD, chk = ((e % PD) / 8) ^ pk_swz(row);
+              const int row = e / D, chk = ((e % D) / 8) ^ pk_swz<D>(row);
               const int32_t kr = keys[row];
               lds_dma16(kb + (int64_t)(kr >= 0 ? kr : 0) * p.sk1 + 8 * chk, kl + b * 512);
             }
-            for (int u = lane + 64 * rbk; u < (kTileKeys / 4) * (PD / 8); u += 64 * RB) {
-              const int bq = u % (PD / 8), a4 = u / (PD / 8);
+            for (int u = lane + 64 * rbk; u < (kTileKeys / 4) * (D / 8); u += 64 * RB) {
+              const int bq = u % (D / 8), a4 = u / (D / 8);
               u32x4_t vr[4];
 #pragma unroll
               for (int s2 = 0; s2 < 4; ++s2) {
@@ -718,7 +758,7 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
               }
             }
           }
-          vm_wait_tile(false);
+          vm_wait_tile<D>(false);
           __syncthreads();
           if (work && it.wave_live) {
             // the list's keys of this lane's S^T elements: slots kblk_base(kb, a) + 0..3, one 16-byte read per block
@@ -746,16 +786,16 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   if (!it.wave_live) return;
   const float lt[2] = {row4_sum(st.l[0]), row4_sum(st.l[1])};
   if (p.n_chunks > 1) {  // partial (O, m, l) of this key chunk for flash_merge_kernel
-    // The fp32 rows pass through this wave's 16 KB of LDS (row r at r * 512 bytes, its 16-byte chunk k in slot
-    // k ^ (r % 16)) so that every global store writes two whole rows, as for the output below.
-    float* fstage = reinterpret_cast<float*>(smem) + wave * (32 * PD);
+    // The fp32 rows pass through this wave's share of LDS (row r at r * 4 D bytes, its 16-byte chunk k in slot
+    // k ^ (r % 16)) so that every global store writes whole rows (two at D = 128), as for the output below.
+    float* fstage = reinterpret_cast<float*>(smem) + wave * (32 * D);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       const int r = 16 * rb + x;
 #pragma unroll
-      for (int db = 0; db < PD / 16; ++db) {
+      for (int db = 0; db < D / 16; ++db) {
         const int k = 4 * db + a;  // d = 4k .. 4k + 3
-        *reinterpret_cast<f32x4_t*>(fstage + r * PD + 4 * (k ^ (r & 15))) = st.o[db][rb];
+        *reinterpret_cast<f32x4_t*>(fstage + r * D + 4 * (k ^ (r & 15))) = st.o[db][rb];
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -763,10 +803,10 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int64_t base0 = ((int64_t)it.chunk * p.BH + it.bh) * p.T + it.rw;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = 2 * i + (lane >> 5), k = lane & 31;
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(fstage + r * PD + 4 * (k ^ (r & 15)));
-      if (it.rw + r < it.T_eff) *reinterpret_cast<f32x4_t*>(p.part_o + (base0 + r) * PD + 4 * k) = v;
+    for (int i = 0; i < D / 8; ++i) {
+      const int r = 256 / D * i + lane / (D / 4), k = lane % (D / 4);
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(fstage + r * D + 4 * (k ^ (r & 15)));
+      if (it.rw + r < it.T_eff) *reinterpret_cast<f32x4_t*>(p.part_o + (base0 + r) * D + 4 * k) = v;
     }
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -778,20 +818,21 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
     }
     return;
   }
-  // The normalised rows pass through this wave's 8 KB of LDS (row r at r * 256 bytes, its 16-byte chunk k in slot
-  // k ^ (r % 16)), so that every global store writes two whole rows: lane l of store i takes bytes 8 (l % 32) .. of
-  // row 2 i + l / 32. Stored from the fragment layout, each store would touch 16 rows.
-  uint16_t* stage = smem + wave * (32 * PD);
+  // The normalised rows pass through this wave's share of LDS (row r at r * 2 D bytes, its 16-byte chunk k in slot
+  // k ^ (r % LPR)), so that every global store writes whole rows (two at D = 128: lane l of store i takes bytes
+  // 8 (l % 32) .. of row 2 i + l / 32; four at 64). Stored from the fragment layout, each store would touch 16 rows.
+  constexpr int LPR = Pipe<D>::LPR;
+  uint16_t* stage = smem + wave * (32 * D);
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
     const float inv = 1.0f / fmaxf(lt[rb], 1.0e-20f);
     const int r = 16 * rb + x;
 #pragma unroll
-    for (int db = 0; db < PD / 16; ++db) {
+    for (int db = 0; db < D / 16; ++db) {
       const int k = 2 * db + (a >> 1);  // 16-byte chunk of d = 16 db + 4 a .. + 3; half a & 1 of it
       const f32x4_t v = st.o[db][rb];
       const u32x2_t w = {pack2<F16>(v[0] * inv, v[1] * inv), pack2<F16>(v[2] * inv, v[3] * inv)};
-      *reinterpret_cast<u32x2_t*>(stage + r * PD + 8 * (k ^ (r & 15)) + 4 * (a & 1)) = w;
+      *reinterpret_cast<u32x2_t*>(stage + r * D + 8 * (k ^ (r & (LPR - 1))) + 4 * (a & 1)) = w;
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -799,9 +840,9 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   uint16_t* obase = p.out + (int64_t)it.bh * p.so0;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = 2 * i + (lane >> 5), q = lane & 31, k = q >> 1;
-    const u32x2_t w = *reinterpret_cast<const u32x2_t*>(stage + r * PD + 8 * (k ^ (r & 15)) + 4 * (q & 1));
+  for (int i = 0; i < D / 8; ++i) {
+    const int r = 256 / D * i + lane / (D / 4), q = lane % (D / 4), k = q >> 1;
+    const u32x2_t w = *reinterpret_cast<const u32x2_t*>(stage + r * D + 8 * (k ^ (r & (LPR - 1))) + 4 * (q & 1));
     const int64_t row = it.rw + r;
     if (row < it.T_eff) *reinterpret_cast<u32x2_t*>(obase + row * p.so1 + 4 * q) = w;
   }
@@ -811,7 +852,9 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
 // LDS tile layouts of the main pass (K tile: pk_off; V^T tile: pv_off), so that the routed phase streams them with
 // direct loads like window tiles. Empty slots (-1, or outside [0, N)) are zero rows. Grid (batches, n_groups, BH),
 // 256 threads.
+template <int D>
 __global__ __launch_bounds__(256) void route_tiles_kernel(FlashParams p, uint16_t* __restrict__ rt) {
+  constexpr int PTE = Pipe<D>::TE, LPR = Pipe<D>::LPR;
   const int b = blockIdx.x, g = blockIdx.y, bh = blockIdx.z, t = threadIdx.x;
   const int batch = bh / p.H;
   const int kvbh = batch * p.Hkv_pb + (bh % p.H) / p.G;
@@ -825,16 +868,17 @@ __global__ __launch_bounds__(256) void route_tiles_kernel(FlashParams p, uint16_
     const int64_t key = slot < p.route_k ? irow[(int64_t)slot * p.si2] : -1;
     return key >= 0 && key < p.N ? key : -1;
   };
-  // K tile: 64 rows x 16 chunks of 16 bytes, 4 per thread
+  // K tile: 64 rows x LPR chunks of 16 bytes, 4 (D = 64: 2) per thread
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int u = t + 256 * i, row = u / 16, chunk = u % 16;
+  for (int i = 0; i < kTileKeys * LPR / 256; ++i) {
+    const int u = t + 256 * i, row = u / LPR, chunk = u % LPR;
     const int64_t key = key_of(row);
     const u32x4_t v = key >= 0 ? ld16(kbase + key * p.sk1 + 8 * chunk) : u32x4_t{0, 0, 0, 0};
-    st16(kt + pk_off(row, chunk), v);
+    st16(kt + pk_off<D>(row, chunk), v);
   }
   // V^T tile: unit (4 keys x 8 d) per thread, transposed into the permuted key order of the V^T layout
-  const int bq = t % (PD / 8), a4 = t / (PD / 8);
+  const int bq = t % LPR, a4 = t / LPR;
+  if (a4 >= kTileKeys / 4) return;
   u32x4_t vr[4];
 #pragma unroll
   for (int s2 = 0; s2 < 4; ++s2) {
@@ -859,49 +903,48 @@ bool flash_pipe_supported(const FlashParams& p, int D, int hpw) {
   // zero) and every V^T offset of one KV head must stay below 4 GiB, so that no offset wraps back into the
   // tensor. Split mode needs whole tiles.
   const int64_t lim = (int64_t)1 << 32;
-  const bool fits = (p.N + kTileKeys) * p.sk1 * 2 < lim && (int64_t)PD * p.np * 2 < lim;
+  const bool fits = (p.N + kTileKeys) * p.sk1 * 2 < lim && (int64_t)D * p.np * 2 < lim;
   const bool chunks_ok = p.n_chunks == 1 || (p.key_chunk % kTileKeys == 0 && p.route_k == 0);
   // 4, 2 or 1 query heads per workgroup; the in-kernel gather of several route groups is built for 4
   const bool heads_ok = (hpw == 4 || hpw == 2 || hpw == 1) && p.G % hpw == 0 &&
                         (hpw == 4 || p.route_k == 0 || p.n_groups == 1);
-  return D == PD && heads_ok && p.key_mask == nullptr && fits && chunks_ok;
+  return (D == 64 || D == 128) && heads_ok && p.key_mask == nullptr && fits && chunks_ok;
 }
 
-size_t route_tiles_bytes(int BH, int n_groups, int route_k) {
+size_t route_tiles_bytes(int BH, int n_groups, int route_k, int D) {
   if (BH <= 0 || n_groups <= 0 || route_k <= 0) return 0;
-  return (size_t)BH * n_groups * ((route_k + kTileKeys - 1) / kTileKeys) * 2 * PTE * sizeof(uint16_t);
+  return (size_t)BH * n_groups * ((route_k + kTileKeys - 1) / kTileKeys) * 2 * kTileKeys * D * sizeof(uint16_t);
 }
 
-hipError_t launch_route_tiles(const FlashParams& p, uint16_t* rt, hipStream_t stream) {
+hipError_t launch_route_tiles(const FlashParams& p, int D, uint16_t* rt, hipStream_t stream) {
   if (p.route_k <= 0) return hipSuccess;
-  hipLaunchKernelGGL(route_tiles_kernel, dim3((unsigned)p.rt_batches, (unsigned)p.n_groups, (unsigned)p.BH), dim3(256),
-                     0, stream, p, rt);
+  const dim3 grid((unsigned)p.rt_batches, (unsigned)p.n_groups, (unsigned)p.BH);
+  if (D == 64) hipLaunchKernelGGL(route_tiles_kernel<64>, grid, dim3(256), 0, stream, p, rt);
+  else hipLaunchKernelGGL(route_tiles_kernel<128>, grid, dim3(256), 0, stream, p, rt);
   return hipGetLastError();
 }
 
-hipError_t launch_flash_pipe(const FlashParams& p, int hpw, hipStream_t stream) {
+namespace {
+template <bool F16, int D>
+hipError_t launch_flash_pipe_t(const FlashParams& p, int hpw, hipStream_t stream) {
   const int64_t items = (int64_t)p.n_kvbh * p.head_splits * p.row_tiles * p.n_chunks;
   if (items <= 0) return hipSuccess;
   if (items > 0x7fffffff) return hipErrorInvalidValue;
   const dim3 grid((unsigned)items), block(64 * PNW);
   const bool gather = p.route_k > 0 && !p.rtiles;
   if (gather && hpw != 4) return hipErrorInvalidValue;
-  if (gather) {
-    if (p.f16) hipLaunchKernelGGL((flash_ping_kernel<true, true, 4>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((flash_ping_kernel<false, true, 4>), grid, block, 0, stream, p);
-  } else if (hpw == 4) {
-    if (p.f16) hipLaunchKernelGGL((flash_ping_kernel<true, false, 4>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((flash_ping_kernel<false, false, 4>), grid, block, 0, stream, p);
-  } else if (hpw == 2) {
-    if (p.f16) hipLaunchKernelGGL((flash_ping_kernel<true, false, 2>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((flash_ping_kernel<false, false, 2>), grid, block, 0, stream, p);
-  } else if (hpw == 1) {
-    if (p.f16) hipLaunchKernelGGL((flash_ping_kernel<true, false, 1>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((flash_ping_kernel<false, false, 1>), grid, block, 0, stream, p);
-  } else {
-    return hipErrorInvalidValue;
-  }
+  if (gather) hipLaunchKernelGGL((flash_ping_kernel<F16, true, 4, D>), grid, block, 0, stream, p);
+  else if (hpw == 4) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 4, D>), grid, block, 0, stream, p);
+  else if (hpw == 2) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 2, D>), grid, block, 0, stream, p);
+  else if (hpw == 1) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 1, D>), grid, block, 0, stream, p);
+  else return hipErrorInvalidValue;
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_flash_pipe(const FlashParams& p, int D, int hpw, hipStream_t stream) {
+  if (D == 64) return p.f16 ? launch_flash_pipe_t<true, 64>(p, hpw, stream) : launch_flash_pipe_t<false, 64>(p, hpw, stream);
+  return p.f16 ? launch_flash_pipe_t<true, 128>(p, hpw, stream) : launch_flash_pipe_t<false, 128>(p, hpw, stream);
 }
 
 }  // namespace bb

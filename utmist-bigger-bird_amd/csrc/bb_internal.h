@@ -29,13 +29,13 @@ struct FlashParams {
 
 hipError_t launch_flash(const FlashParams& p, int D, int hpw, bool split, hipStream_t stream);
 hipError_t launch_flash_merge(const FlashParams& p, int D, hipStream_t stream);
-// Software-pipelined main-pass kernel (head_dim 128, kv_groups % 4 == 0, no token mask, 64-aligned route groups).
+// Software-pipelined main-pass kernel (head_dim 64 or 128, no token mask).
 // The pipelined kernel with hpw query heads per workgroup (4, 2 or 1; the schedule's rows per tile 32 x 8 / hpw).
 bool flash_pipe_supported(const FlashParams& p, int D, int hpw);
-hipError_t launch_flash_pipe(const FlashParams& p, int hpw, hipStream_t stream);
+hipError_t launch_flash_pipe(const FlashParams& p, int D, int hpw, hipStream_t stream);
 // Bytes of the pre-gathered routed tiles of one call, and the kernel that writes them (p.rtiles) for the main pass.
-size_t route_tiles_bytes(int BH, int n_groups, int route_k);
-hipError_t launch_route_tiles(const FlashParams& p, uint16_t* rt, hipStream_t stream);
+size_t route_tiles_bytes(int BH, int n_groups, int route_k, int D);
+hipError_t launch_route_tiles(const FlashParams& p, int D, uint16_t* rt, hipStream_t stream);
 hipError_t launch_transpose_v(const uint16_t* v, int64_t sv0, int64_t sv1, int n_kvbh, int64_t N, int64_t np, int D,
                               uint16_t* vt, hipStream_t stream);
 
