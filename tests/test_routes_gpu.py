@@ -133,3 +133,43 @@ def test_mfma_scores_match_reference_order(name, T, scale_q, scale_k, dev, monke
     torch.cuda.synchronize()
     assert torch.equal(pooled.cpu(), pooled_ref.cpu()), f"{name}: pooled values differ"
     assert torch.equal(idx.cpu(), idx_ref.cpu()), f"{name}: route indices differ"
+
+
+@pytest.mark.parametrize("T,H,Hkv,d,nr,dtype", [
+    (129, 8, 2, 64, 64, torch.bfloat16), (4097, 8, 8, 64, 64, torch.bfloat16), (4099, 8, 4, 64, 64, torch.bfloat16),
+    (5000, 16, 2, 64, 64, torch.bfloat16), (3001, 16, 2, 128, 64, torch.bfloat16),   # 512 rows: two row blocks
+    (2049, 4, 4, 128, 64, torch.float16), (2047, 8, 4, 128, 64, torch.float16), (131, 8, 8, 64, 40, torch.float16),
+    (3000, 16, 2, 64, 64, torch.float16), (1030, 8, 4, 32, 64, torch.float16)])
+def test_score_workgroups_bit_exact(T, H, Hkv, d, nr, dtype, dev):
+    """Every scorer instantiation (head_dim 64 on MFMA; fp16 workgroups of 64, 128 and 256 rows) at the edges of its key
+    chunks, bit for bit against the oracle."""
+    print(f"case score_workgroups T={T} {H}/{Hkv} d={d} nr={nr} {dtype}", flush=True)
+    sink, window, budget = 8, 64, 32
+    inp = make_inputs(T, H, Hkv, d, seed=T, window=window, sink=sink, dtype=dtype)
+    q, k = inp["q"], inp["k"]
+    idx, pooled = hip_routes(q.to(dev), k.to(dev), num_heads=H, num_kv_heads=Hkv, sink=sink, window=window, budget=budget,
+                             n_route=nr, scaling=d ** -0.5, return_pooled=True)
+    r = min(nr, T)
+    want, want_pooled = oracle.routes(q[0], k[0], sink=sink, window=window, budget=budget, scaling=d ** -0.5, n_route=nr,
+                                      route_pool="mean", qpos=torch.arange(T - r, T), return_pooled=True)
+    assert torch.equal(idx.cpu(), want)
+    prob = (want_pooled.double() * 2.0 ** -40 / r).float()
+    assert torch.equal(pooled.cpu()[:, sink:T - window], prob[:, sink:T - window])
+
+
+@pytest.mark.parametrize("heads", [(32, 8), (32, 16), (32, 32)], ids=["gqa4", "gqa2", "mha"])
+def test_mfma_scores_d64_match_reference_order(heads, dev, monkeypatch):
+    """head_dim 64 on MFMA with exact fix-up against every score in the reference order, rows and keys over many binades."""
+    (H, Hkv), T, d = heads, 16384, 64
+    print(f"case mfma_scores_d64 {H}/{Hkv}", flush=True)
+    inp = make_inputs(T, H, Hkv, d, seed=12, sink=64, window=4096, device=dev, rng="device")
+    g = torch.Generator(device=dev).manual_seed(3)
+    q = inp["q"] * torch.exp2(torch.randint(-12, 8, (1, H, T, 1), device=dev, generator=g).to(inp["q"].dtype))
+    k = inp["k"] * torch.exp2(torch.randint(-12, 8, (1, Hkv, T, 1), device=dev, generator=g).to(inp["k"].dtype))
+    k[:, :, 1000:1100] = 0
+    kw = dict(num_heads=H, num_kv_heads=Hkv, sink=64, window=4096, budget=512, scaling=d ** -0.5, return_pooled=True)
+    idx, pooled = hip_routes(q, k, **kw)
+    monkeypatch.setenv("BB_ROUTES_REFERENCE_ORDER", "1")
+    idx_ref, pooled_ref = hip_routes(q, k, **kw)
+    monkeypatch.delenv("BB_ROUTES_REFERENCE_ORDER")
+    assert torch.equal(pooled.cpu(), pooled_ref.cpu()) and torch.equal(idx.cpu(), idx_ref.cpu())

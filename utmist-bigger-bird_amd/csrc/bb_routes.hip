@@ -37,10 +37,11 @@ namespace bb {
 namespace {
 
 constexpr int kScoreKeys = 32;    // keys per scores_kernel block (8 key groups of 4)
-constexpr int kScoreIters = 16;   // fewest key blocks per scores workgroup (RouteGeom::iters: 16, 32, 64 or 128)
+constexpr int kScoreIters = 4;    // fewest key blocks per scores workgroup (RouteGeom::iters: 4 to 128)
+constexpr int kCus = 256;
 constexpr int kSumKeys = 1024;    // keys per rowsum_kernel workgroup
 constexpr int kPoolKeys = 512;    // keys per pooled_kernel workgroup (2 per thread)
-constexpr int kMaxRows = 256;     // route rows (G * r) per scores_kernel workgroup (more rows use more row blocks)
+constexpr int kMaxRows = 256;     // most route rows (G * r) per scores workgroup (more rows use more row blocks)
 constexpr float kFixOne = 1099511627776.0f;  // 2^40
 
 BB_DEV uint64_t fix40(float v) { return (uint64_t)(v * kFixOne); }
@@ -66,45 +67,47 @@ struct RouteGeom {
   int64_t ns;  // score row stride: n rounded up to 8 (16-byte aligned rows)
 };
 
-// Scores: one workgroup = up to 256 route rows of one KV head x g.iters blocks of kScoreKeys keys.
-// Q^T stays in LDS for the whole key range; each key block is staged as fp32 K^T. Thread t owns rows
-// 8*(t%32)..+7 and keys 4*(t/32)..+3 of a block. Every score is built in the reference's accumulation order: per
+// Scores: one workgroup = up to ROWS route rows of one KV head x the keys of g.iters blocks of kScoreKeys, in steps of
+// KEYS = 8192 / ROWS (32 keys against 256 rows; 64 and 128 against the 128 and 64 rows of a group of 2 and 1 query
+// heads, whose threads would otherwise compute rows that do not exist). Q^T stays in LDS for the whole key range; each
+// step's keys are staged as fp32 K^T. Thread t owns rows 8*(t%(ROWS/8))..+7 and keys 4*(t/(ROWS/8))..+3 of a step. Every score is built in the reference's accumulation order: per
 // 32-element block of d, two sequential fp32 chains over the even and the odd elements (fmaf of two bf16 values is
 // one rounding of the exact product sum), then acc = acc + (even + odd); for fp16 inputs (F16) one sequential chain
 // over d (an fp16 product is exact in fp32 as well) and the result rounded to fp16.
 // LDS of scores_kernel. bf16: K^T staged in fp32 (the chains take fp32 operands). fp16: K^T kept in fp16 (the FMAs take
 // fp16 operands directly) and the row-max partials share its space after the last block, so that two workgroups fit
 // a CU (74 KB each at head_dim 128).
-template <int D, bool F16>
+template <int D, bool F16, int ROWS>
 struct ScoresSmem {
-  uint16_t qs[D][kMaxRows];                              // Q^T (16-bit)
-  float ks[D][kScoreKeys + 4];                           // K^T (fp32), padded rows
-  float rmax_part[kMaxRows][kScoreKeys / 4 + 1];
+  uint16_t qs[D][ROWS];                                  // Q^T (16-bit)
+  float ks[D][8192 / ROWS + 4];                          // K^T (fp32), padded rows
+  float rmax_part[ROWS][2048 / ROWS + 1];
 };
-template <int D>
-struct ScoresSmem<D, true> {
-  uint16_t qs[D][kMaxRows];
+template <int D, int ROWS>
+struct ScoresSmem<D, true, ROWS> {
+  uint16_t qs[D][ROWS];
   union {
-    uint16_t ks[D][kScoreKeys + 8];                      // K^T (fp16), padded rows
-    float rmax_part[kMaxRows][kScoreKeys / 4 + 1];       // after the last block
+    uint16_t ks[D][8192 / ROWS + 8];                     // K^T (fp16), padded rows
+    float rmax_part[ROWS][2048 / ROWS + 1];              // after the last step
   };
 };
 
-template <int D, bool F16>
+template <int D, bool F16, int ROWS>
 __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g, float* __restrict__ pmax) {
   static_assert(D % 32 == 0, "head_dim must be a multiple of 32");
-  __shared__ __attribute__((aligned(16))) ScoresSmem<D, F16> sm;
+  constexpr int KEYS = 8192 / ROWS, RG = ROWS / 8;
+  __shared__ __attribute__((aligned(16))) ScoresSmem<D, F16, ROWS> sm;
   auto& qs = sm.qs;
   auto& ks = sm.ks;
   auto& rmax_part = sm.rmax_part;
   const int tid = threadIdx.x;
   const int kchunk = blockIdx.x, rblk = blockIdx.y, bkv = blockIdx.z;
   const int batch = bkv / p.Hkv, kvh = bkv % p.Hkv;
-  const int row0 = rblk * kMaxRows;
-  const int nrows = g.rows - row0 < kMaxRows ? g.rows - row0 : kMaxRows;
+  const int row0 = rblk * ROWS;
+  const int nrows = g.rows - row0 < ROWS ? g.rows - row0 : ROWS;
 
   // stage Q^T: row -> (head slot, query i)
-  for (int e = tid; e < kMaxRows * (D / 8); e += 256) {
+  for (int e = tid; e < ROWS * (D / 8); e += 256) {
     const int row = e / (D / 8), c8 = e % (D / 8);
     u32x4_t v = {0, 0, 0, 0};
     if (row < nrows) {
@@ -119,7 +122,7 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
     }
   }
 
-  const int rg = tid & 31, kg = tid >> 5;
+  const int rg = tid % RG, kg = tid / RG;
   int64_t qp[8];
 #pragma unroll
   for (int a = 0; a < 8; ++a) {
@@ -132,29 +135,30 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
   const uint16_t* kbase = p.k + (int64_t)bkv * p.sk0;
   uint16_t* srow_base = p.scores + (int64_t)bkv * g.rows * g.ns;
 
-  // K blocks: thread t holds the 16-byte units t, t + 256, ... of a block; the next block's loads are in flight
-  // while the current one is scored
-  constexpr int KPT = (kScoreKeys * (D / 8) + 255) / 256;
+  // K steps: thread t holds the 16-byte units t, t + 256, ... of a step; the next step's loads are in flight while the
+  // current one is scored
+  constexpr int KPT = (KEYS * (D / 8) + 255) / 256;
+  const int steps = g.iters * kScoreKeys / KEYS;  // g.iters is a multiple of 4
   auto kload = [&](int it, u32x4_t (&dst)[KPT]) {
-    const int64_t jb = ((int64_t)kchunk * g.iters + it) * kScoreKeys;
+    const int64_t jb = (int64_t)kchunk * g.iters * kScoreKeys + (int64_t)it * KEYS;
 #pragma unroll
     for (int u = 0; u < KPT; ++u) {
       const int e = tid + 256 * u;
       const int64_t j = jb + e / (D / 8);
-      dst[u] = e < kScoreKeys * (D / 8) && j < p.n ? ld16(kbase + j * p.sk1 + 8 * (e % (D / 8))) : u32x4_t{0, 0, 0, 0};
+      dst[u] = e < KEYS * (D / 8) && j < p.n ? ld16(kbase + j * p.sk1 + 8 * (e % (D / 8))) : u32x4_t{0, 0, 0, 0};
     }
   };
   u32x4_t knext[KPT];
   kload(0, knext);
 
-  for (int it = 0; it < g.iters; ++it) {
-    const int64_t j0 = ((int64_t)kchunk * g.iters + it) * kScoreKeys;
+  for (int it = 0; it < steps; ++it) {
+    const int64_t j0 = (int64_t)kchunk * g.iters * kScoreKeys + (int64_t)it * KEYS;
     if (j0 >= p.n) break;
     __syncthreads();  // previous block's K^T fully consumed (and Q^T staged on the first pass)
 #pragma unroll
     for (int u = 0; u < KPT; ++u) {
       const int e = tid + 256 * u;
-      if (e < kScoreKeys * (D / 8)) {
+      if (e < KEYS * (D / 8)) {
         const int key = e / (D / 8), c8 = e % (D / 8);
         const u32x4_t v = knext[u];
 #pragma unroll
@@ -170,7 +174,7 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
       }
     }
     __syncthreads();
-    if (it + 1 < g.iters) kload(it + 1, knext);
+    if (it + 1 < steps) kload(it + 1, knext);
 
     float acc[8][4];
 #pragma unroll
@@ -254,13 +258,13 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
   if (tid < nrows) {
     float mx = rmax_part[tid][0];
 #pragma unroll
-    for (int b = 1; b < kScoreKeys / 4; ++b) mx = fmaxf(mx, rmax_part[tid][b]);
+    for (int b = 1; b < KEYS / 4; ++b) mx = fmaxf(mx, rmax_part[tid][b]);
     pmax[((int64_t)bkv * g.n_kb1 + kchunk) * g.rows + row0 + tid] = mx;
   }
 }
 
-// MFMA scores with exact fix-up (head_dim 128). The bf16 score of every (route row, key) must be the one the
-// reference order above produces. Both that order and the MFMA path sum the same 128 exact bf16 products
+// MFMA scores with exact fix-up (head_dim 128 or 64; the counts below are those of 128). The bf16 score of every (route
+// row, key) must be the one the reference order above produces. Both that order and the MFMA path sum the same exact bf16 products
 // p_d = q_d k_d in fp32, and each result's distance from the exact sum is bounded per product (u = 2^-24; every
 // rounding of a partial sum x errs by at most u |x|, and |x| <= the sum of |p_d| over the products in it):
 //   * reference order, d = 32 c + 2 t + parity: the even / odd chain of block c rounds at its steps t' = 1..15 (step 0
@@ -272,13 +276,16 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
 //     32 u M_s + 2 u sum_s|p|, with M_s = max over the slice of |p_d| <= max|q_d| max|k_d|; the eight slice partials
 //     are then added in order, so slice s passes through 8 - max(s, 1) more roundings.
 // So |reference - MFMA| <= u (sum_d c_d |q_d| |k_d| + 32 sum_s max_s|q| max_s|k|) with
-// c_d = (16 - max(t, 1)) + 1 + (4 - max(c, 1)) + (10 - max(s, 1)). One accumulating MFMA chain computes that bound
+// c_d = (16 - max(t, 1)) + 1 + (4 - max(c, 1)) + (10 - max(s, 1)) (head_dim 64: 2 blocks and 4 slices, so 2 and 6 in
+// place of 4 and 10). One accumulating MFMA chain computes that bound
 // per score: |K| against the weighted row c_d |q_d| (rounded up to bf16), then one more MFMA of the per-slice maxima
 // of |K| against 32 x the per-slice maxima of |Q|. The bound's own MFMA rounding (all terms are non-negative; below
 // 2^-16 relative), the fp32 evaluation of the bound and second-order terms are covered by the factor 1 + 2^-10 in
 // kScoreSlack, underflow by the absolute 2^-100. If s - B and s + B round to the same bf16 value, so does the
 // reference-order score (it is an fp32 value in [s - B, s + B]), and that value is taken; otherwise (a score near a
 // rounding boundary, or tiny) the score is recomputed in the reference order.
+//
+// At head_dim 64 the same scheme replaced the VALU scorer: bb_routes over 20011 tokens, 32 heads over 8, 250 -> 148 us.
 //
 // Workgroup: one KV head, up to 256 route rows (G r), g.iters blocks of 32 keys; 8 waves, wave w owns rows
 // 32w..32w+31 (one MFMA block, Q^T operands in registers; two waves per SIMD hide each other's MFMA and LDS
@@ -287,14 +294,20 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
 // the scores: a few wave-iterations per block for the whole workgroup, instead of one per wave). Scores go through an
 // LDS tile per wave so that fix-ups land before one coalesced store, made at the start of the next block.
 constexpr float kScoreSlack = 5.9662e-8f;  // u (1 + 2^-10)
-constexpr int kMsRowPitch = 136;           // bf16 elements per staged Q row (272 bytes: conflict-free row reads)
+template <int D>
+constexpr int kMsRowPitch = D + 8;         // bf16 elements per staged Q row (16 bytes past it: conflict-free row reads)
 constexpr int kMsTilePitch = 40;           // bf16 per score-tile row (80 bytes: conflict-free 8-byte row writes)
 
-// Weight c_d of the certification bound for element d of a 128-element dot product (see above).
+// Weight c_d of the certification bound for element d of a D-element dot product (see above).
+template <int D>
 BB_DEV int bound_weight(int d) {
   const int c = d >> 5, t = (d & 31) >> 1, s = d >> 4;
-  return (16 - (t > 1 ? t : 1)) + 1 + (4 - (c > 1 ? c : 1)) + (10 - (s > 1 ? s : 1));
+  return (16 - (t > 1 ? t : 1)) + 1 + (D / 32 - (c > 1 ? c : 1)) + (2 + D / 16 - (s > 1 ? s : 1));
 }
+// 16-byte chunk c of staged key j sits in slot c ^ ms_swz(j) of its row: the fragment reads (32 keys, one chunk) then
+// touch every bank slot once per 16-lane group (at D = 64 a row is half of the slots, so keys of one parity share a half).
+template <int D>
+BB_DEV int ms_swz(int j) { return D == 128 ? (j & 15) : ((j >> 1) & 7); }
 
 // Magnitude maximum of the eight bf16 values of a fragment (abs bit patterns order as unsigned integers).
 typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
@@ -309,11 +322,12 @@ BB_DEV uint32_t abs_max8(u32x4_t a) {
 // rows, so their workgroups are 2 or 4 waves and no wave computes rows that do not exist)
 template <int D, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void scores_mfma_kernel(RoutesParams p, RouteGeom g, float* __restrict__ pmax) {
-  static_assert(D == 128, "MFMA scores are built for head_dim 128");
-  static_assert(NW == 2 || NW == 4 || NW == 8, "K staging splits 512 16-byte pieces evenly over the threads");
-  constexpr int ROWS = 32 * NW, NT = 64 * NW, KPT = kScoreKeys * (D / 8) / NT;  // K pieces per thread
-  __shared__ __attribute__((aligned(16))) uint16_t qs[ROWS][kMsRowPitch];   // Q rows (bf16)
-  __shared__ __attribute__((aligned(16))) uint16_t kt[kScoreKeys][D];       // K block, chunk c of key j at c ^ (j % 16)
+  static_assert(D == 64 || D == 128, "MFMA scores are built for head_dim 64 and 128");
+  static_assert(NW == 2 || NW == 4 || NW == 8, "2, 4 or 8 waves");
+  constexpr int CPR = D / 8, PIECES = kScoreKeys * CPR;  // 16-byte pieces per key and per K block
+  constexpr int ROWS = 32 * NW, NT = 64 * NW, KPT = (PIECES + NT - 1) / NT;  // pieces per thread
+  __shared__ __attribute__((aligned(16))) uint16_t qs[ROWS][kMsRowPitch<D>];  // Q rows (bf16)
+  __shared__ __attribute__((aligned(16))) uint16_t kt[kScoreKeys][D];       // K block, chunk c of key j at c ^ ms_swz(j)
   __shared__ __attribute__((aligned(16))) float kf[kScoreKeys][D];          // the same block in fp32 (same slots)
   __shared__ __attribute__((aligned(16))) uint16_t st[NW][32][kMsTilePitch];  // per-wave score tile (bf16)
   __shared__ uint16_t flist[NW * 32 * kScoreKeys];                          // fix-ups: wave << 10 | lane << 4 | r
@@ -359,7 +373,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
       for (int hw = 0; hw < 2; ++hw) {
         const float a = __uint_as_float(((qf[dk][w] >> (16 * hw)) & 0x7fffu) << 16);
-        const float v = a * (float)bound_weight(16 * dk + 8 * h + 2 * w + hw);  // exact: <= 13 significant bits
+        const float v = a * (float)bound_weight<D>(16 * dk + 8 * h + 2 * w + hw);  // exact: <= 13 significant bits
         packed |= ((__float_as_uint(v) + 0xffffu) >> 16) << (16 * hw);          // rounded up to bf16
       }
       qw[dk][w] = packed;
@@ -387,14 +401,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     }
   };
 
-  // K blocks: piece e = tid + NT x (key e / 16, chunk e % 16) is 16 bytes; the next block's load is in flight while
+  // K blocks: piece e = tid + NT x (key e / CPR, chunk e % CPR) is 16 bytes; the next block's load is in flight while
   // the current one is processed
   auto kload = [&](int it, u32x4_t (&dst)[KPT]) {
 #pragma unroll
     for (int x = 0; x < KPT; ++x) {
       const int e = tid + NT * x;
-      const int64_t j = ((int64_t)kchunk * g.iters + it) * kScoreKeys + (e >> 4);
-      dst[x] = j < p.n ? ld16(kbase + j * p.sk1 + 8 * (e & 15)) : u32x4_t{0, 0, 0, 0};
+      const int64_t j = ((int64_t)kchunk * g.iters + it) * kScoreKeys + e / CPR;
+      dst[x] = e < PIECES && j < p.n ? ld16(kbase + j * p.sk1 + 8 * (e % CPR)) : u32x4_t{0, 0, 0, 0};
     }
   };
   u32x4_t knext[KPT];
@@ -409,8 +423,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     if (tid == 0) fcount = 0u;
 #pragma unroll
     for (int x = 0; x < KPT; ++x) {  // stage the K block: bf16 for the MFMA fragments, fp32 for the fix-ups
-      const int e = tid + NT * x, skey = e >> 4, schunk = e & 15;
-      const int slot = 8 * (schunk ^ (skey & 15));  // chunk c of key j in slot c ^ (j % 16)
+      const int e = tid + NT * x, skey = e / CPR, schunk = e % CPR;
+      if (PIECES % NT != 0 && e >= PIECES) break;
+      const int slot = 8 * (schunk ^ ms_swz<D>(skey));
       const u32x4_t v = knext[x];
       *reinterpret_cast<u32x4_t*>(&kt[skey][slot]) = v;
       *reinterpret_cast<f32x4_t*>(&kf[skey][slot]) = f32x4_t{
@@ -429,7 +444,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     uint32_t mk[D / 16];  // max |k| over this lane's half of slice dk (key li)
 #pragma unroll
     for (int dk = 0; dk < D / 16; ++dk) {
-      const u32x4_t kv = *reinterpret_cast<const u32x4_t*>(&kt[li][8 * ((2 * dk + h) ^ (li & 15))]);
+      const u32x4_t kv = *reinterpret_cast<const u32x4_t*>(&kt[li][8 * ((2 * dk + h) ^ ms_swz<D>(li))]);
       const f32x16_t cur = mfma32(as_bf16x8(kv), as_bf16x8(qf[dk]), f32x16_t{});
       const u32x4_t ka = kv & kAbs;
       aac = mfma32(as_bf16x8(ka), as_bf16x8(qw[dk]), aac);
@@ -443,7 +458,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     {  // + 32 sum_s max_s|k| max_s|q|: slice maxima of key li (both halves) at positions 0..7 of the h = 0 lane
       u32x4_t mka = {0, 0, 0, 0};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < D / 32; ++i) {
         const uint32_t x = mk[2 * i] | (mk[2 * i + 1] << 16);
         const auto sw = __builtin_amdgcn_permlane32_swap(x, x, false, false);
         const u16x2_t m = __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, sw[0]), __builtin_bit_cast(u16x2_t, sw[1]));
@@ -503,7 +518,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
       const int lrow = el & 31, kk = 8 * (er >> 2) + 4 * (el >> 5) + (er & 3);
       const uint16_t* qr = qs[32 * ew + lrow];
       const float* kr = kf[kk];
-      const int ksw = kk & 15;  // chunk c of key kk sits at slot c ^ (kk % 16)
+      const int ksw = ms_swz<D>(kk);  // chunk c of key kk sits at slot c ^ ksw
       float accx = 0.0f;
 #pragma unroll
       for (int blk = 0; blk < D / 32; ++blk) {
@@ -1107,16 +1122,19 @@ hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, uin
   const int nbkv = p.B * p.Hkv;
   const dim3 sgrid(g.n_kb1, g.row_blocks, nbkv);
   // fp16 scores (8x finer rounding than bf16) are computed in the reference order directly
-  if (p.f16)
-    hipLaunchKernelGGL((scores_kernel<D, true>), sgrid, dim3(256), 0, stream, p, g, pmax);
-  else if (D == 128 && !p.scores_reference_order) {
+  if (p.f16) {
+    if (g.rows <= 64) hipLaunchKernelGGL((scores_kernel<D, true, 64>), sgrid, dim3(256), 0, stream, p, g, pmax);
+    else if (g.rows <= 128) hipLaunchKernelGGL((scores_kernel<D, true, 128>), sgrid, dim3(256), 0, stream, p, g, pmax);
+    else hipLaunchKernelGGL((scores_kernel<D, true, kMaxRows>), sgrid, dim3(256), 0, stream, p, g, pmax);
+  } else if (D >= 64 && !p.scores_reference_order) {
+    constexpr int MD = D >= 64 ? D : 64;  // head_dim 32 has no MFMA instantiation
     const int nw = g.rows <= 64 ? 2 : (g.rows <= 128 ? 4 : 8);  // waves of 32 rows per workgroup
     const dim3 mgrid(g.n_kb1, (g.rows + 32 * nw - 1) / (32 * nw), nbkv);
-    if (nw == 2) hipLaunchKernelGGL((scores_mfma_kernel<128, 2>), mgrid, dim3(128), 0, stream, p, g, pmax);
-    else if (nw == 4) hipLaunchKernelGGL((scores_mfma_kernel<128, 4>), mgrid, dim3(256), 0, stream, p, g, pmax);
-    else hipLaunchKernelGGL((scores_mfma_kernel<128, 8>), mgrid, dim3(512), 0, stream, p, g, pmax);
+    if (nw == 2) hipLaunchKernelGGL((scores_mfma_kernel<MD, 2>), mgrid, dim3(128), 0, stream, p, g, pmax);
+    else if (nw == 4) hipLaunchKernelGGL((scores_mfma_kernel<MD, 4>), mgrid, dim3(256), 0, stream, p, g, pmax);
+    else hipLaunchKernelGGL((scores_mfma_kernel<MD, 8>), mgrid, dim3(512), 0, stream, p, g, pmax);
   } else
-    hipLaunchKernelGGL((scores_kernel<D, false>), sgrid, dim3(256), 0, stream, p, g, pmax);
+    hipLaunchKernelGGL((scores_kernel<D, false, kMaxRows>), sgrid, dim3(256), 0, stream, p, g, pmax);
   hipLaunchKernelGGL(rowmax_kernel, dim3(g.rows, nbkv), dim3(64), 0, stream, p, g, pmax);
   if (p.f16) hipLaunchKernelGGL(rowsum_kernel<true>, dim3(g.n_kb2, nbkv, g.sum_splits), dim3(256), 0, stream, p, g, psum);
   else hipLaunchKernelGGL(rowsum_kernel<false>, dim3(g.n_kb2, nbkv, g.sum_splits), dim3(256), 0, stream, p, g, psum);
@@ -1137,21 +1155,23 @@ hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, uin
   return hipGetLastError();
 }
 
-RouteGeom geom(int64_t n, int H, int Hkv, int B, int r) {
+RouteGeom geom(int64_t n, int H, int Hkv, int B, int r, bool f16) {
   RouteGeom g;
   g.G = H / Hkv;
   g.rows = g.G * r;
   g.row_blocks = (g.rows + kMaxRows - 1) / kMaxRows;
-  // Longer key chunks per scores workgroup while the grid keeps at least 256 workgroups (one per CU): each workgroup
-  // stages its Q rows and bound weights once, so fewer, longer workgroups spend less on that (128K routes, interleaved
-  // A/B: 0.885 ms with 16 blocks, 0.812 with 64, 0.793 with 128; the scores are the same)
+  // Key blocks per scores workgroup: as many as make one round of resident workgroups (one, two or four per CU by LDS:
+  // 8, 4 and 2 waves; two, two and three of the VALU workgroups that fp16 scores run on), since every workgroup stages
+  // its Q rows and bound weights once, but not fewer than 4 and at most 128, in multiples of 4 (a step of the VALU
+  // scorer is up to 128 keys). At 128K tokens that is 128 blocks (0.793 ms against 0.885 with 16); with 16 at the least
+  // short prompts left half of the CUs idle: whole bb_routes calls of 32 heads over 8, 2048 tokens 120 -> 76 us, 8192
+  // 132 -> 105, 8111 in fp16 293 -> 171.
   const int64_t nbkv = (int64_t)(B > 0 ? B : 1) * Hkv;
-  g.iters = kScoreIters;
-  while (g.iters < 128) {
-    const int64_t chunks = (n + kScoreKeys * 2 * g.iters - 1) / (kScoreKeys * 2 * g.iters);
-    if (chunks * g.row_blocks * nbkv < 256) break;
-    g.iters *= 2;
-  }
+  const int per_cu = g.rows > 128 ? (f16 ? 2 : 1) : (g.rows > 64 ? 2 : 4);
+  const int64_t blocks32 = (n + kScoreKeys - 1) / kScoreKeys, lanes = nbkv * g.row_blocks;
+  const int64_t chunks = kCus * per_cu / lanes > 1 ? kCus * per_cu / lanes : 1;
+  const int64_t it = ((blocks32 + chunks - 1) / chunks + 3) & ~(int64_t)3;
+  g.iters = (int)(it < kScoreIters ? kScoreIters : (it > 128 ? 128 : it));
   g.n_kb1 = (int)((n + kScoreKeys * g.iters - 1) / (kScoreKeys * g.iters));
   g.n_kb2 = (int)((n + kSumKeys - 1) / kSumKeys);
   g.ns = (n + 7) & ~(int64_t)7;
@@ -1230,7 +1250,7 @@ hipError_t launch_topk_rows(const uint64_t* keys, int rows, int64_t stride, int6
 }
 
 size_t routes_workspace_bytes(int64_t n, int H, int Hkv, int B, int r) {
-  RouteGeom g = geom(n, H, Hkv, B, r);
+  RouteGeom g = geom(n, H, Hkv, B, r, true);  // fp16 scores have at least as many key chunks as bf16 ones
   const size_t nbkv = (size_t)B * Hkv;
   size_t s = 0;
   s += align256(nbkv * g.rows * (size_t)g.ns * 2);        // scores
@@ -1246,7 +1266,7 @@ size_t routes_workspace_bytes(int64_t n, int H, int Hkv, int B, int r) {
 
 hipError_t launch_routes(RoutesParams& p, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (ws_bytes < routes_workspace_bytes(p.n, p.H, p.Hkv, p.B, p.r)) return hipErrorInvalidValue;
-  RouteGeom g = geom(p.n, p.H, p.Hkv, p.B, p.r);
+  RouteGeom g = geom(p.n, p.H, p.Hkv, p.B, p.r, p.f16 != 0);
   const size_t nbkv = (size_t)p.B * p.Hkv;
   p.pstride = p.n;
   p.n_dev = nullptr;
