@@ -359,8 +359,8 @@ __global__ __launch_bounds__(64 * NW, 1) void flash_kernel(FlashParams p) {
   }
 }
 
-// Combine split partials: one wave per (head, row); lanes cover D. Chunks that hold no key of the row are skipped (the
-// split kernels write none for a workgroup of such rows). The chunks' (max, sum) pairs are read by
+// Combine split partials: one wave per (head, row); lanes cover D. Chunks that hold no key of the row are skipped (their
+// partials are empty or not written). The chunks' (max, sum) pairs are read by
 // one lane each, 64 at a time, and the partial rows eight at a time, so the latency is that of a few round trips and
 // does not grow with the chunk count.
 template <bool F16, int D>

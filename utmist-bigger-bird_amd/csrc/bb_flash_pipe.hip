@@ -553,7 +553,9 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   // split mode (exact tail: no routes): only the tiles of key chunk `chunk`, [c0, c1)
   int64_t c0 = 0, c1 = w1 > f1 ? w1 : f1;
   if (p.n_chunks > 1) {
-    if (chunk_unused(p, chunk, qlo, qhi)) return;  // the merge skips it
+    // A chunk without a tile of these rows runs no step and writes an empty partial, which the merge does not read: an
+    // early return here, before or after the loop, changed the code of the whole kernel (main pass 24.19 -> 24.27 ms,
+    // tail 0.413 -> 0.425 ms at 128K).
     c0 = (int64_t)chunk * p.key_chunk / kTileKeys;
     const int64_t ce = ((int64_t)chunk + 1) * p.key_chunk / kTileKeys;
     if (ce < c1) c1 = ce;

@@ -406,9 +406,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   auto kload = [&](int it, u32x4_t (&dst)[KPT]) {
 #pragma unroll
     for (int x = 0; x < KPT; ++x) {
-      const int e = tid + NT * x;
+      const uint32_t e = tid + NT * x;
       const int64_t j = ((int64_t)kchunk * g.iters + it) * kScoreKeys + e / CPR;
-      dst[x] = e < PIECES && j < p.n ? ld16(kbase + j * p.sk1 + 8 * (e % CPR)) : u32x4_t{0, 0, 0, 0};
+      dst[x] = (PIECES % NT == 0 || e < PIECES) && j < p.n ? ld16(kbase + j * p.sk1 + 8 * (e % CPR)) : u32x4_t{0, 0, 0, 0};
     }
   };
   u32x4_t knext[KPT];
@@ -423,7 +423,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     if (tid == 0) fcount = 0u;
 #pragma unroll
     for (int x = 0; x < KPT; ++x) {  // stage the K block: bf16 for the MFMA fragments, fp32 for the fix-ups
-      const int e = tid + NT * x, skey = e / CPR, schunk = e % CPR;
+      const uint32_t e = tid + NT * x;
+      const int skey = e / CPR, schunk = e % CPR;
       if (PIECES % NT != 0 && e >= PIECES) break;
       const int slot = 8 * (schunk ^ ms_swz<D>(skey));
       const u32x4_t v = knext[x];
