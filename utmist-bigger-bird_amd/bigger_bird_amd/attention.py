@@ -207,7 +207,7 @@ class RDAttention(nn.Module):
         if getattr(k, "turbo", None) is not None:      # compressed KV cache handle, one decode token
             return k.attend(q, self.scaling)
         if t == n:
-            none = torch.full((self.num_heads, 1, 1), -1, dtype=torch.int32, device=q.device)
+            none = torch.empty((self.num_heads, 1, 0), dtype=torch.int32, device=q.device)  # no route slots
             return bigger_bird_flash(q[0], k[0], v[0], none, front=0, window=n, num_heads=self.num_heads,
                                      kv_groups=self.groups, scale=self.scaling)[None]
         if t == 1 and self.head_dim in (64, 128) and self.groups in (1, 2, 4, 8):
@@ -272,7 +272,7 @@ class RDAttention(nn.Module):
                                 route_chunk=chunk, row_end=n - r, vt=vt, **flash)
         if r:
             # Final r queries attend exactly (window = n): written straight into the output rows.
-            none = torch.full((bh, 1, 1), -1, dtype=torch.int32, device=q.device)
+            none = torch.empty((bh, 1, 0), dtype=torch.int32, device=q.device)  # no route slots
             bigger_bird_flash(Q[:, n - r:], K, V, none, front=0, window=n, token_mask=None, route_chunk=None, vt=vt,
                               out=out[:, n - r:], **flash)
         return out.unflatten(0, (bsz, self.num_heads))

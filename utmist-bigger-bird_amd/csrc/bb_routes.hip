@@ -16,10 +16,8 @@
 //
 // Kernels (all on the caller's stream, no host synchronisation):
 //   scores_kernel   scores of G*r route rows against a 256-key range, bf16 to the workspace, partial row max
-//   rowmax_kernel   partial maxima -> row max
-//   rowsum_kernel   fixed-point partial row sums over 1024-key blocks
-//   invz_kernel     partial sums -> fp32 scale 2^40 / Z per row
-//   pooled_kernel   per (head, key): pooled fixed-point probability over the r rows
+//   rowsum_kernel   row max from the partials, then fixed-point row sums over 1024-key blocks (integer atomics: any order)
+//   pooled_kernel   per (head, key): pooled fixed-point probability over the r rows, scaled by 2^40 / Z of each row
 //   topk_*_kernel   top-budget per head: log-linear histogram over many workgroups, the threshold bin, compaction of
 //                   the keys above it and of its candidates, exact choice among the candidates (value desc, index asc)
 //                   and ascending emission through a bitmap; an MSD radix select over the whole range when the
@@ -65,6 +63,8 @@ struct RouteGeom {
   int iters;  // key blocks of kScoreKeys per scores workgroup: n_kb1 = ceil(n / (kScoreKeys iters))
   int sum_rows, sum_splits;  // rowsum_kernel: rows per workgroup (a multiple of 4) and row slices
   int64_t ns;  // score row stride: n rounded up to 8 (16-byte aligned rows)
+  uint32_t* top_hist;  // [B * H][kTopBins] and [B * H][kTopMetaWords]: cleared by the scorer for the top-k kernels
+  uint32_t* top_meta;
 };
 
 // Scores: one workgroup = up to ROWS route rows of one KV head x the keys of g.iters blocks of kScoreKeys, in steps of
@@ -92,6 +92,17 @@ struct ScoresSmem<D, true, ROWS> {
   };
 };
 
+// What the later kernels accumulate into, cleared by the scorer's workgroups of the first key chunk: the row sums of
+// their rows, and (row block 0) the top-k histograms and list counters of the KV head's query heads.
+BB_DEV void clear_row_state(const RoutesParams& p, const RouteGeom& g, int bkv, int rblk, int row0, int nrows, int nt) {
+  for (int e = threadIdx.x; e < nrows; e += nt) p.rowsum[(int64_t)bkv * g.rows + row0 + e] = 0;
+  if (rblk == 0) {
+    const int64_t head0 = (int64_t)(bkv / p.Hkv) * p.H + (int64_t)(bkv % p.Hkv) * g.G;
+    for (int e = threadIdx.x; e < g.G * kTopBins; e += nt) g.top_hist[head0 * kTopBins + e] = 0u;
+    for (int e = threadIdx.x; e < g.G * kTopMetaWords; e += nt) g.top_meta[head0 * kTopMetaWords + e] = 0u;
+  }
+}
+
 template <int D, bool F16, int ROWS>
 __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g, float* __restrict__ pmax) {
   static_assert(D % 32 == 0, "head_dim must be a multiple of 32");
@@ -105,6 +116,7 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
   const int batch = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int row0 = rblk * ROWS;
   const int nrows = g.rows - row0 < ROWS ? g.rows - row0 : ROWS;
+  if (kchunk == 0) clear_row_state(p, g, bkv, rblk, row0, nrows, 256);
 
   // stage Q^T: row -> (head slot, query i)
   for (int e = tid; e < ROWS * (D / 8); e += 256) {
@@ -259,7 +271,7 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
     float mx = rmax_part[tid][0];
 #pragma unroll
     for (int b = 1; b < KEYS / 4; ++b) mx = fmaxf(mx, rmax_part[tid][b]);
-    pmax[((int64_t)bkv * g.n_kb1 + kchunk) * g.rows + row0 + tid] = mx;
+    pmax[((int64_t)bkv * g.rows + row0 + tid) * g.n_kb1 + kchunk] = mx;
   }
 }
 
@@ -339,6 +351,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   const int batch = bkv / p.Hkv, kvh = bkv % p.Hkv;
   const int row0 = rblk * ROWS;
   const int nrows = g.rows - row0 < ROWS ? g.rows - row0 : ROWS;
+  if (kchunk == 0) clear_row_state(p, g, bkv, rblk, row0, nrows, NT);
 
   // stage Q rows: row -> (head slot, route query i)
   for (int e = tid; e < ROWS * (D / 8); e += NT) {
@@ -552,19 +565,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     if (h == 0 && myrow < nrows) {
       const uint32_t fk = rmax_fix[myrow];
       const float fx = fk ? ordered_to_float(fk) : -__builtin_huge_valf();
-      pmax[((int64_t)bkv * g.n_kb1 + kchunk) * g.rows + row0 + myrow] = fmaxf(mx, fx);
+      pmax[((int64_t)bkv * g.rows + row0 + myrow) * g.n_kb1 + kchunk] = fmaxf(mx, fx);
     }
   }
-}
-
-// One wave per (KV head, route row): lanes stride over the key-block partials, then a wave maximum.
-__global__ __launch_bounds__(64) void rowmax_kernel(RoutesParams p, RouteGeom g, const float* __restrict__ pmax) {
-  const int row = blockIdx.x, bkv = blockIdx.y, lane = threadIdx.x;
-  float mx = -__builtin_huge_valf();
-  for (int kb = lane; kb < g.n_kb1; kb += 64) mx = fmaxf(mx, pmax[((int64_t)bkv * g.n_kb1 + kb) * g.rows + row]);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-  if (lane == 0) p.rowmax[(int64_t)bkv * g.rows + row] = __float_as_uint(mx);
 }
 
 // fix40(det_exp2(y) * scale) as an integer-valued float below 2^41, for y <= 0 (or -inf / NaN) and 0 < scale <= 1,
@@ -586,11 +589,16 @@ BB_DEV float fix40_exp2(float y, float scale) {
   return truncf(ldexpf(q * scale, (int)(n + 40.0f)));
 }
 
-// Fixed-point partial row sums: one wave per row (4 rows in flight per workgroup), 16 keys per lane. The rows of a
-// key block may be cut into blockIdx.z slices of g.sum_rows rows, so short sequences still fill the chip. The terms
-// are integers below 2^41, so their sums stay exact in double precision (1024 terms per workgroup row < 2^51).
+// Row maxima and fixed-point row sums: one wave per row (4 rows in flight per workgroup), 16 keys per lane. The rows of a
+// key block may be cut into blockIdx.z slices of g.sum_rows rows, so short sequences still fill the chip. The workgroup
+// first reduces its rows' maxima from the scorer's partials, four lanes per row, into LDS (key block 0 stores them for
+// pooled_kernel). The terms are integers below 2^41, so their sums stay exact in double precision (1024 terms per
+// workgroup row < 2^51), and the 64-bit integer atomics that add them up over the key blocks give the same bits in any
+// order. (The maximum and the reciprocal of the sum used to be launches of their own, 5 us each.)
 template <bool F16>
-__global__ __launch_bounds__(256) void rowsum_kernel(RoutesParams p, RouteGeom g, uint64_t* __restrict__ psum) {
+__global__ __launch_bounds__(256) void rowsum_kernel(RoutesParams p, RouteGeom g, const float* __restrict__ pmax) {
+  extern __shared__ unsigned long long row_sum[];  // [g.sum_rows], then the rows' maxima
+  float* row_max = reinterpret_cast<float*>(row_sum + g.sum_rows);
   const int kb = blockIdx.x, bkv = blockIdx.y;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r_begin = blockIdx.z * g.sum_rows;
@@ -603,8 +611,22 @@ __global__ __launch_bounds__(256) void rowsum_kernel(RoutesParams p, RouteGeom g
     na = ld16(src);
     nb = ld16(src + 8);
   }
+  for (int r0 = r_begin; r0 < r_end; r0 += 64) {  // four lanes per row; the first rows' score loads are in flight
+    const int row = r0 + (int)(threadIdx.x >> 2);
+    const float* pm = pmax + ((int64_t)bkv * g.rows + (row < r_end ? row : r_end - 1)) * g.n_kb1;
+    float mx = -__builtin_huge_valf();
+#pragma unroll 8
+    for (int i = threadIdx.x & 3; i < g.n_kb1; i += 4) mx = fmaxf(mx, pm[i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 1));
+    mx = fmaxf(mx, __shfl_xor(mx, 2));
+    if (row < r_end && (threadIdx.x & 3) == 0) {
+      row_max[row - r_begin] = mx;
+      if (kb == 0) p.rowmax[(int64_t)bkv * g.rows + row] = __float_as_uint(mx);
+    }
+  }
+  __syncthreads();
   for (int row = r_begin + wave; row < r_end; row += 4) {
-    const float M = __uint_as_float(p.rowmax[(int64_t)bkv * g.rows + row]);
+    const float M = row_max[row - r_begin];
     const uint16_t* src = p.scores + ((int64_t)bkv * g.rows + row) * g.ns + j0;
     double acc = 0.0;
     if (j0 + 16 <= p.n) {
@@ -628,51 +650,37 @@ __global__ __launch_bounds__(256) void rowsum_kernel(RoutesParams p, RouteGeom g
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-    if (lane == 0) psum[((int64_t)bkv * g.n_kb2 + kb) * g.rows + row] = (uint64_t)acc;
+    if (lane == 0) row_sum[row - r_begin] = (unsigned long long)acc;
   }
-}
-
-// One wave per (KV head, route row): integer partial sums (order-free), then 2^40 / Z. The workgroups of the first G
-// rows of each KV head also clear that query head's top-k histogram and list counters, which the top-k kernels
-// accumulate into.
-__global__ __launch_bounds__(64) void invz_kernel(RoutesParams p, RouteGeom g, const uint64_t* __restrict__ psum,
-                                                 float* __restrict__ invz, uint32_t* __restrict__ top_hist,
-                                                 uint32_t* __restrict__ top_meta) {
-  const int row = blockIdx.x, bkv = blockIdx.y, lane = threadIdx.x;
-  if (row < g.G) {
-    const int head = (bkv / p.Hkv) * p.H + (bkv % p.Hkv) * g.G + row;
-    for (int b = lane; b < kTopBins; b += 64) top_hist[(int64_t)head * kTopBins + b] = 0u;
-    if (lane < kTopMetaWords) top_meta[kTopMetaWords * head + lane] = 0u;
-  }
-  uint64_t z = 0;
-  for (int kb = lane; kb < g.n_kb2; kb += 64) z += psum[((int64_t)bkv * g.n_kb2 + kb) * g.rows + row];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) z += __shfl_xor(z, off);
-  if (lane == 0) {
-    const int64_t t = (int64_t)bkv * g.rows + row;
-    p.rowsum[t] = z;
-    invz[t] = (float)(1099511627776.0 / (double)z);
-  }
+  __syncthreads();
+  // one atomic per row, 64 rows to an instruction (issued by each wave after its row they cost 17 us at 128K tokens)
+  unsigned long long* sums = reinterpret_cast<unsigned long long*>(p.rowsum) + (int64_t)bkv * g.rows;
+  for (int row = r_begin + (int)threadIdx.x; row < r_end; row += 256) atomicAdd(sums + row, row_sum[row - r_begin]);
 }
 
 // Pooled fixed-point probability per (query head, key): two consecutive keys per thread (one 4-byte score load per
 // route row, eight rows' loads in flight), the head's r rows in a loop, sums exact in double precision (64 rows x
-// 2^41 < 2^53).
+// 2^41 < 2^53). The rows' maxima and 2^40 / Z are staged in LDS first (r pairs).
 template <bool F16>
-__global__ __launch_bounds__(256) void pooled_kernel(RoutesParams p, RouteGeom g, const float* __restrict__ invz) {
+__global__ __launch_bounds__(256) void pooled_kernel(RoutesParams p, RouteGeom g) {
+  extern __shared__ __attribute__((aligned(8))) float mz[];  // [r][2]: maximum, 2^40 / Z
   const int64_t j0 = 2 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
   const int head = blockIdx.y;  // over B * H
-  if (j0 >= p.n) return;
   const int batch = head / p.H, hh = head % p.H;
   const int kvh = hh / g.G, hs = hh % g.G;
   const int64_t bkv = (int64_t)batch * p.Hkv + kvh;
+  for (int i = threadIdx.x; i < p.r; i += 256) {
+    const int64_t t = bkv * g.rows + (int64_t)hs * p.r + i;
+    mz[2 * i] = __uint_as_float(p.rowmax[t]);
+    mz[2 * i + 1] = (float)(1099511627776.0 / (double)p.rowsum[t]);
+  }
+  __syncthreads();
+  if (j0 >= p.n) return;
   const int64_t lo = p.sink, hi = p.n - p.window;  // eligible keys [lo, hi)
   double P0 = 0.0, P1 = 0.0;
   if (j0 + 2 > lo && j0 < hi) {
     // keys past n read as -inf: score rows end at g.ns, a multiple of 8, and the scorer stores -inf there
     const uint16_t* src = p.scores + (bkv * g.rows + (int64_t)hs * p.r) * g.ns + j0;
-    const float* mrow = reinterpret_cast<const float*>(p.rowmax) + bkv * g.rows + (int64_t)hs * p.r;
-    const float* zrow = invz + bkv * g.rows + (int64_t)hs * p.r;
     int i = 0;
     for (; i < p.r; i += 8) {
       const int nb = p.r - i < 8 ? p.r - i : 8;
@@ -682,7 +690,7 @@ __global__ __launch_bounds__(256) void pooled_kernel(RoutesParams p, RouteGeom g
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         if (u >= nb) break;
-        const float M = mrow[i + u], iz = zrow[i + u];
+        const float M = mz[2 * (i + u)], iz = mz[2 * (i + u) + 1];
         const float x0 = score_f32<F16>((uint16_t)(w[u] & 0xffffu)) * p.scaling;
         const float x1 = score_f32<F16>((uint16_t)(w[u] >> 16)) * p.scaling;
         const double f0 = (double)fix40_exp2((x0 - M) * kLog2e, iz);
@@ -850,7 +858,7 @@ __device__ __forceinline__ void topk_radix_head(const RoutesParams& p, int head)
   }
 }
 
-// Fast top-budget selection in three launches (all heads at once):
+// Fast top-budget selection in three launches (all heads at once; one launch, topk_small_kernel, for short ranges):
 //   topk_hist_kernel     many workgroups per head: log-linear histogram of the keys (bin = 32 x bit length + the 5
 //                        bits after the leading one, 0 for zero; for float keys 32 bins per octave of the value),
 //                        monotone in the key. Decode routing fills it in its pool kernel instead.
@@ -903,14 +911,15 @@ __global__ __launch_bounds__(256) void topk_hist_kernel(RoutesParams p, TopWs w)
     if (h[b]) atomicAdd(&w.hist[(int64_t)head * kTopBins + b], h[b]);
 }
 
-// The bin b* that holds the budget-th largest key of one head, from its histogram (all 256 threads of the workgroup
+// The bin b* that holds the budget-th largest key of one head, from its histogram (all NT threads of the workgroup
 // call it): above = keys in higher bins, need = budget - above. With fewer keys than the budget, b* = 0 and every
 // key is taken (need = the zero keys).
 struct TopPick {
   int bstar, above, need;
 };
+template <int NT>
 BB_DEV TopPick top_pick(const uint32_t* __restrict__ hist, uint32_t budget, uint32_t* part, TopPick* s_pick) {
-  constexpr int PER = (kTopBins + 255) / 256;  // bins per thread, taken from the top
+  constexpr int PER = (kTopBins + NT - 1) / NT;  // bins per thread, taken from the top
   const int tid = threadIdx.x;
   uint32_t c[PER], sum = 0;
 #pragma unroll
@@ -921,7 +930,7 @@ BB_DEV TopPick top_pick(const uint32_t* __restrict__ hist, uint32_t budget, uint
   }
   if (tid == 0) *s_pick = TopPick{-1, 0, 0};
   uint32_t total;
-  const uint32_t incl = block_incl_scan<256>(sum, part, total);  // over threads, top bins first
+  const uint32_t incl = block_incl_scan<NT>(sum, part, total);  // over threads, top bins first
   const uint32_t before = incl - sum;
   if (before < budget && incl >= budget) {  // the budget-th largest key lies in this thread's bins
     uint32_t cum = before;
@@ -962,7 +971,7 @@ __global__ __launch_bounds__(256) void topk_compact_kernel(RoutesParams p, TopWs
     const int64_t t = t0 + 256 * k + tid;
     v[k] = t < cnt ? P[t] : 0;
   }
-  const TopPick pk = top_pick(w.hist + (int64_t)head * kTopBins, (uint32_t)p.budget, part, &s_pick);
+  const TopPick pk = top_pick<256>(w.hist + (int64_t)head * kTopBins, (uint32_t)p.budget, part, &s_pick);
   TopMeta* m = w.meta + head;
   if (blockIdx.x == 0 && tid == 0) {
     m->bstar = pk.bstar;
@@ -1019,93 +1028,79 @@ __global__ __launch_bounds__(256) void topk_compact_kernel(RoutesParams p, TopWs
   }
 }
 
-__global__ __launch_bounds__(kTopThreads) void topk_final_kernel(RoutesParams p, TopWs w) {
-  __shared__ uint64_t cv[kTopCand];
-  __shared__ int32_t ci[kTopCand];
-  __shared__ uint32_t bits[kTopBitmapBits / 32];
-  __shared__ uint32_t scan[kTopThreads / 64];
-  __shared__ uint32_t sub[kTopSub];
-  __shared__ int16_t tie_list[kTopCand];
-  __shared__ int s_sub[3];  // s*, candidates still needed from s*, length of the s* list
-  const int head = blockIdx.x, tid = threadIdx.x;
-  int64_t lo, cnt;
-  top_range(p, lo, cnt);
-  const TopMeta m = w.meta[head];
-  if (m.ncand > (uint32_t)kTopCand || cnt > kTopBitmapBits) {
-    topk_radix_head(p, head);
-    return;
-  }
-  const int nc = (int)m.ncand;
-  const int words = (int)((cnt + 31) / 32);
-  for (int i = tid; i < nc; i += kTopThreads) {
-    cv[i] = w.candv[(int64_t)head * kTopCand + i];
-    ci[i] = w.candi[(int64_t)head * kTopCand + i];
-  }
-  for (int i = tid; i < words; i += kTopThreads) bits[i] = 0u;
-  __syncthreads();
+struct TopFinalLds {
+  uint64_t cv[kTopCand];
+  int32_t ci[kTopCand];
+  uint32_t bits[kTopBitmapBits / 32];
+  uint32_t scan[kTopThreads / 64];
+  uint32_t sub[kTopSub];
+  int16_t tie_list[kTopCand];
+  int s_sub[3];  // s*, candidates still needed from s*, length of the s* list
+};
+
+// The choice among the nc candidates L.cv / L.ci (the keys of bin pk.bstar) and the ascending emission of every key
+// marked in L.bits (the caller has marked the keys above that bin). All kTopThreads threads call it, after a barrier.
+BB_DEV void topk_choose(const RoutesParams& p, int head, int64_t lo, int64_t cnt, int nc, const TopPick& pk, TopFinalLds& L) {
+  const int tid = threadIdx.x, words = (int)((cnt + 31) / 32);
   // Chosen candidates: fewer than `need` others beat them (larger value, or equal value and lower index). Inside
   // bin b* the next 10 bits of the key order the candidates further (top_sub_key): a histogram of those finds the
   // sub-bin s* of the need-th largest candidate; candidates above s* are chosen, and only the ones in s* are ranked
   // against each other. The clamped float bins (their keys span several octaves) rank every candidate instead.
   const bool fk = p.float_keys != 0;
-  const bool refine = !(fk && (m.bstar == 1 || m.bstar == kTopBins - 1));
-  int need2 = m.need, sstar = -1;
+  const bool refine = !(fk && (pk.bstar == 1 || pk.bstar == kTopBins - 1));
+  int need2 = pk.need, sstar = -1;
   if (refine) {
-    for (int i = tid; i < kTopSub; i += kTopThreads) sub[i] = 0u;
+    for (int i = tid; i < kTopSub; i += kTopThreads) L.sub[i] = 0u;
     if (tid == 0) {  // need = 0 (every key above b*): no sub-bin, nothing more to choose
-      s_sub[0] = kTopSub;
-      s_sub[1] = 0;
-      s_sub[2] = 0;
+      L.s_sub[0] = kTopSub;
+      L.s_sub[1] = 0;
+      L.s_sub[2] = 0;
     }
     __syncthreads();
-    for (int i = tid; i < nc; i += kTopThreads) atomicAdd(&sub[top_sub_key(cv[i], fk)], 1u);
+    for (int i = tid; i < nc; i += kTopThreads) atomicAdd(&L.sub[top_sub_key(L.cv[i], fk)], 1u);
     __syncthreads();
     // thread t owns sub-bin kTopSub - 1 - t (top first): inclusive scan of the counts
-    const uint32_t c = sub[kTopSub - 1 - tid];
+    const uint32_t c = L.sub[kTopSub - 1 - tid];
     uint32_t tot;
-    const uint32_t incl = block_incl_scan<kTopThreads>(c, scan, tot);
-    if (incl - c < (uint32_t)m.need && incl >= (uint32_t)m.need) {
-      s_sub[0] = kTopSub - 1 - tid;
-      s_sub[1] = m.need - (int)(incl - c);
+    const uint32_t incl = block_incl_scan<kTopThreads>(c, L.scan, tot);
+    if (incl - c < (uint32_t)pk.need && incl >= (uint32_t)pk.need) {
+      L.s_sub[0] = kTopSub - 1 - tid;
+      L.s_sub[1] = pk.need - (int)(incl - c);
     }
     __syncthreads();
-    sstar = s_sub[0];
-    need2 = s_sub[1];
+    sstar = L.s_sub[0];
+    need2 = L.s_sub[1];
     // candidates above s* are chosen; the ones in s* go to a short list
     for (int i = tid; i < nc; i += kTopThreads) {
-      const int sk = top_sub_key(cv[i], fk);
-      if (sk > sstar) atomicOr(&bits[(ci[i] - lo) >> 5], 1u << ((ci[i] - lo) & 31));
-      else if (sk == sstar) tie_list[atomicAdd(&s_sub[2], 1)] = i;
+      const int sk = top_sub_key(L.cv[i], fk);
+      if (sk > sstar) atomicOr(&L.bits[(L.ci[i] - lo) >> 5], 1u << ((L.ci[i] - lo) & 31));
+      else if (sk == sstar) L.tie_list[atomicAdd(&L.s_sub[2], 1)] = i;
     }
     __syncthreads();
   }
-  const int nr = refine ? s_sub[2] : nc;
+  const int nr = refine ? L.s_sub[2] : nc;
   for (int r = tid; r < nr; r += kTopThreads) {
-    const int i = refine ? tie_list[r] : r;
-    const uint64_t v = cv[i];
-    const int32_t ix = ci[i];
+    const int i = refine ? L.tie_list[r] : r;
+    const uint64_t v = L.cv[i];
+    const int32_t ix = L.ci[i];
     int rank = 0;
     for (int q = 0; q < nr; ++q) {
-      const int j = refine ? tie_list[q] : q;
-      rank += (cv[j] > v) || (cv[j] == v && ci[j] < ix);
+      const int j = refine ? L.tie_list[q] : q;
+      rank += (L.cv[j] > v) || (L.cv[j] == v && L.ci[j] < ix);
     }
-    if (rank < need2) atomicOr(&bits[(ix - lo) >> 5], 1u << ((ix - lo) & 31));
-  }
-  for (uint32_t i = tid; i < m.nsel; i += kTopThreads) {
-    const int32_t ix = w.sel[(int64_t)head * p.pstride + i];
-    atomicOr(&bits[(ix - lo) >> 5], 1u << ((ix - lo) & 31));
+    if (rank < need2) atomicOr(&L.bits[(ix - lo) >> 5], 1u << ((ix - lo) & 31));
   }
   __syncthreads();
   // ascending emission: each thread a contiguous run of words, exclusive scan of their bit counts
   const int per = (words + kTopThreads - 1) / kTopThreads;
   const int w0 = tid * per, w1 = w0 + per < words ? w0 + per : words;
   uint32_t mine = 0;
-  for (int x = w0; x < w1; ++x) mine += __builtin_popcount(bits[x]);
+  for (int x = w0; x < w1; ++x) mine += __builtin_popcount(L.bits[x]);
   uint32_t chosen;
-  uint32_t pos = block_incl_scan<kTopThreads>(mine, scan, chosen) - mine;
+  uint32_t pos = block_incl_scan<kTopThreads>(mine, L.scan, chosen) - mine;
   int32_t* out = p.out_idx + (int64_t)head * p.budget;
   for (int x = w0; x < w1; ++x) {
-    uint32_t b = bits[x];
+    uint32_t b = L.bits[x];
     while (b) {
       const int bit = __builtin_ctz(b);
       b &= b - 1;
@@ -1117,9 +1112,86 @@ __global__ __launch_bounds__(kTopThreads) void topk_final_kernel(RoutesParams p,
   for (uint32_t i = chosen + tid; i < (uint32_t)p.budget; i += kTopThreads) out[i] = -1;
 }
 
+__global__ __launch_bounds__(kTopThreads) void topk_final_kernel(RoutesParams p, TopWs w) {
+  __shared__ TopFinalLds L;
+  const int head = blockIdx.x, tid = threadIdx.x;
+  int64_t lo, cnt;
+  top_range(p, lo, cnt);
+  const TopMeta m = w.meta[head];
+  if (m.ncand > (uint32_t)kTopCand || cnt > kTopBitmapBits) {
+    topk_radix_head(p, head);
+    return;
+  }
+  const int nc = (int)m.ncand;
+  const int words = (int)((cnt + 31) / 32);
+  for (int i = tid; i < nc; i += kTopThreads) {
+    L.cv[i] = w.candv[(int64_t)head * kTopCand + i];
+    L.ci[i] = w.candi[(int64_t)head * kTopCand + i];
+  }
+  for (int i = tid; i < words; i += kTopThreads) L.bits[i] = 0u;
+  __syncthreads();
+  for (uint32_t i = tid; i < m.nsel; i += kTopThreads) {
+    const int32_t ix = w.sel[(int64_t)head * p.pstride + i];
+    atomicOr(&L.bits[(ix - lo) >> 5], 1u << ((ix - lo) & 31));
+  }
+  topk_choose(p, head, lo, cnt, nc, TopPick{m.bstar, m.above, m.need}, L);
+}
+
+// The whole selection of one head in one workgroup, for eligible ranges of up to kTopSmall keys (16 per thread, kept in
+// registers): histogram, threshold bin and candidate list in LDS, then topk_choose. One launch in place of three that
+// take 6-8 us each whatever their size (8111 tokens, 32 heads: 22 -> 9.7 us).
+constexpr int kTopSmall = 16 * kTopThreads;
+__global__ __launch_bounds__(kTopThreads) void topk_small_kernel(RoutesParams p) {
+  constexpr int PER = kTopSmall / kTopThreads;
+  __shared__ TopFinalLds L;
+  __shared__ uint32_t hist[kTopBins];
+  __shared__ TopPick s_pick;
+  __shared__ uint32_t ncand;
+  const int head = blockIdx.x, tid = threadIdx.x;
+  int64_t lo, cnt;
+  top_range(p, lo, cnt);
+  const bool fk = p.float_keys != 0;
+  const uint64_t* P = p.pooled + (int64_t)head * p.pstride + lo;
+  uint64_t v[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int t = kTopThreads * k + tid;
+    v[k] = t < cnt ? P[t] : 0;
+  }
+  for (int b = tid; b < kTopBins; b += kTopThreads) hist[b] = 0u;
+  for (int i = tid; i < (int)((cnt + 31) / 32); i += kTopThreads) L.bits[i] = 0u;
+  if (tid == 0) ncand = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if (kTopThreads * k + tid < cnt) atomicAdd(&hist[top_bin(v[k], fk)], 1u);
+  __syncthreads();
+  const TopPick pk = top_pick<kTopThreads>(hist, (uint32_t)p.budget, L.scan, &s_pick);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int t = kTopThreads * k + tid;
+    if (t >= cnt) continue;
+    const int bin = top_bin(v[k], fk);
+    if (bin > pk.bstar) {
+      atomicOr(&L.bits[t >> 5], 1u << (t & 31));
+    } else if (bin == pk.bstar) {
+      const uint32_t c = atomicAdd(&ncand, 1u);
+      if (c < (uint32_t)kTopCand) {
+        L.cv[c] = v[k];
+        L.ci[c] = (int32_t)(lo + t);
+      }
+    }
+  }
+  __syncthreads();
+  if (ncand > (uint32_t)kTopCand) {  // heavy ties
+    topk_radix_head(p, head);
+    return;
+  }
+  topk_choose(p, head, lo, cnt, (int)ncand, pk, L);
+}
+
 template <int D>
-hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, uint64_t* psum, float* invz,
-                           const TopWs& tw, hipStream_t stream) {
+hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, const TopWs& tw, hipStream_t stream) {
   const int nbkv = p.B * p.Hkv;
   const dim3 sgrid(g.n_kb1, g.row_blocks, nbkv);
   // fp16 scores (8x finer rounding than bf16) are computed in the reference order directly
@@ -1136,19 +1208,22 @@ hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, uin
     else hipLaunchKernelGGL((scores_mfma_kernel<MD, 8>), mgrid, dim3(512), 0, stream, p, g, pmax);
   } else
     hipLaunchKernelGGL((scores_kernel<D, false, kMaxRows>), sgrid, dim3(256), 0, stream, p, g, pmax);
-  hipLaunchKernelGGL(rowmax_kernel, dim3(g.rows, nbkv), dim3(64), 0, stream, p, g, pmax);
-  if (p.f16) hipLaunchKernelGGL(rowsum_kernel<true>, dim3(g.n_kb2, nbkv, g.sum_splits), dim3(256), 0, stream, p, g, psum);
-  else hipLaunchKernelGGL(rowsum_kernel<false>, dim3(g.n_kb2, nbkv, g.sum_splits), dim3(256), 0, stream, p, g, psum);
-  hipLaunchKernelGGL(invz_kernel, dim3(g.rows, nbkv), dim3(64), 0, stream, p, g, psum, invz, tw.hist,
-                     reinterpret_cast<uint32_t*>(tw.meta));
+  const unsigned sshm = (unsigned)((sizeof(uint64_t) + sizeof(float)) * g.sum_rows);
+  if (p.f16) hipLaunchKernelGGL(rowsum_kernel<true>, dim3(g.n_kb2, nbkv, g.sum_splits), dim3(256), sshm, stream, p, g, pmax);
+  else hipLaunchKernelGGL(rowsum_kernel<false>, dim3(g.n_kb2, nbkv, g.sum_splits), dim3(256), sshm, stream, p, g, pmax);
   const dim3 pgrid((unsigned)((p.n + kPoolKeys - 1) / kPoolKeys), p.B * p.H);
-  if (p.f16) hipLaunchKernelGGL(pooled_kernel<true>, pgrid, dim3(256), 0, stream, p, g, invz);
-  else hipLaunchKernelGGL(pooled_kernel<false>, pgrid, dim3(256), 0, stream, p, g, invz);
+  const unsigned pshm = (unsigned)(2 * sizeof(float) * p.r);
+  if (p.f16) hipLaunchKernelGGL(pooled_kernel<true>, pgrid, dim3(256), pshm, stream, p, g);
+  else hipLaunchKernelGGL(pooled_kernel<false>, pgrid, dim3(256), pshm, stream, p, g);
   if (p.budget > 0) {
     int64_t lo = p.sink < p.n ? (p.sink > 0 ? p.sink : 0) : p.n, hi = p.n - p.window < p.n ? p.n - p.window : p.n;
     const int64_t cnt = hi > lo ? hi - lo : 0;
     const unsigned chunks = (unsigned)((cnt + kTopChunk - 1) / kTopChunk);
     const int heads = p.B * p.H;
+    if (cnt <= kTopSmall) {
+      hipLaunchKernelGGL(topk_small_kernel, dim3(heads), dim3(kTopThreads), 0, stream, p);
+      return hipGetLastError();
+    }
     hipLaunchKernelGGL(topk_hist_kernel, dim3(chunks, heads), dim3(256), 0, stream, p, tw);
     hipLaunchKernelGGL(topk_compact_kernel, dim3(chunks, heads), dim3(256), 0, stream, p, tw);
     hipLaunchKernelGGL(topk_final_kernel, dim3(heads), dim3(kTopThreads), 0, stream, p, tw);
@@ -1203,7 +1278,7 @@ TopWs carve_top_ws(char* w, int64_t n, size_t heads) {
   return t;
 }
 
-// Clears the histograms and counters that the top-k kernels accumulate into (pooled_kernel does it for prefill).
+// Clears the histograms and counters that the top-k kernels accumulate into (the scorer does it for prefill).
 __global__ __launch_bounds__(256) void topk_clear_kernel(TopWs w) {
   const int row = blockIdx.x;
   for (int b = threadIdx.x; b < kTopBins; b += 256) w.hist[(int64_t)row * kTopBins + b] = 0u;
@@ -1241,6 +1316,10 @@ hipError_t launch_topk_rows(const uint64_t* keys, int rows, int64_t stride, int6
   const int64_t lo = front > 0 ? front : 0;
   const int64_t cnt = stride > lo ? stride - lo : 0;
   const unsigned chunks = (unsigned)((cnt + kTopChunk - 1) / kTopChunk);
+  if (cnt <= kTopSmall) {  // whatever the device length: the range is at most cnt
+    hipLaunchKernelGGL(topk_small_kernel, dim3(rows), dim3(kTopThreads), 0, stream, p);
+    return hipGetLastError();
+  }
   if (!(flags & kTopHistReady)) {
     hipLaunchKernelGGL(topk_clear_kernel, dim3(rows), dim3(256), 0, stream, tw);
     if (chunks > 0) hipLaunchKernelGGL(topk_hist_kernel, dim3(chunks, rows), dim3(256), 0, stream, p, tw);
@@ -1257,9 +1336,7 @@ size_t routes_workspace_bytes(int64_t n, int H, int Hkv, int B, int r) {
   s += align256(nbkv * g.rows * (size_t)g.ns * 2);        // scores
   s += align256(nbkv * g.n_kb1 * g.rows * 4);             // partial max
   s += align256(nbkv * g.rows * 4);                       // row max
-  s += align256(nbkv * g.n_kb2 * g.rows * 8);             // partial sums
   s += align256(nbkv * g.rows * 8);                       // row sums
-  s += align256(nbkv * g.rows * 4);                       // 2^40 / Z
   s += align256((size_t)B * H * (size_t)n * 8);           // pooled
   s += top_ws_bytes(n, (size_t)B * H);
   return s;
@@ -1276,15 +1353,15 @@ hipError_t launch_routes(RoutesParams& p, void* ws, size_t ws_bytes, hipStream_t
   p.scores = reinterpret_cast<uint16_t*>(w); w += align256(nbkv * g.rows * (size_t)g.ns * 2);
   float* pmax = reinterpret_cast<float*>(w); w += align256(nbkv * g.n_kb1 * g.rows * 4);
   p.rowmax = reinterpret_cast<uint32_t*>(w); w += align256(nbkv * g.rows * 4);
-  uint64_t* psum = reinterpret_cast<uint64_t*>(w); w += align256(nbkv * g.n_kb2 * g.rows * 8);
   p.rowsum = reinterpret_cast<uint64_t*>(w); w += align256(nbkv * g.rows * 8);
-  float* invz = reinterpret_cast<float*>(w); w += align256(nbkv * g.rows * 4);
   p.pooled = reinterpret_cast<uint64_t*>(w); w += align256((size_t)p.B * p.H * (size_t)p.n * 8);
   const TopWs tw = carve_top_ws(w, p.n, (size_t)p.B * p.H);
+  g.top_hist = tw.hist;
+  g.top_meta = reinterpret_cast<uint32_t*>(tw.meta);
   switch (p.D) {
-    case 32: return launch_routes_d<32>(p, g, pmax, psum, invz, tw, stream);
-    case 64: return launch_routes_d<64>(p, g, pmax, psum, invz, tw, stream);
-    case 128: return launch_routes_d<128>(p, g, pmax, psum, invz, tw, stream);
+    case 32: return launch_routes_d<32>(p, g, pmax, tw, stream);
+    case 64: return launch_routes_d<64>(p, g, pmax, tw, stream);
+    case 128: return launch_routes_d<128>(p, g, pmax, tw, stream);
     default: return hipErrorInvalidValue;
   }
 }
