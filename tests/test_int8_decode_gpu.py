@@ -66,6 +66,29 @@ def _check(got, ref, what):
 
 
 # 32769 and 131329 keys: 128 splits of 257 / 1027 keys (not a multiple of the 32-key chunk), the last one short
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("size,min_scale", [(1.0, 1e-4), (1e-3, 1e-4), (1e-6, 1e-20), (1e4, 1e-4)])
+def test_quantize_near_halves(size, min_scale, dtype, dev):
+    """Rows full of values within a few ulps of (k + 1/2) scale, where the reciprocal and the division could round to
+    different integers: bit for bit rint(x / scale) with numpy's correctly rounded fp32 division."""
+    import numpy as np
+
+    print(f"case quantize_near_halves {dtype} size={size} min_scale={min_scale}", flush=True)
+    g = torch.Generator().manual_seed(7)
+    rows, d = 20000, 128
+    amax = (torch.rand(rows, 1, generator=g) + 0.5) * size
+    x = (torch.randint(-126, 126, (rows, d), generator=g) + 0.5) * (amax / 127)
+    x = x * (1 + (torch.randint(-3, 4, (rows, d), generator=g) * 2.0 ** -23))
+    x[:, :1] = amax
+    x[::5] = torch.randn(rows // 5, d, generator=g) * size
+    x = x.to(dtype)
+    q, s = quantize(x.to(dev), scale_dtype=torch.float32, min_scale=min_scale)
+    f = x.float().numpy()
+    want_s = np.maximum(np.abs(f).max(1, keepdims=True) / np.float32(127), np.float32(min_scale))
+    want_q = np.clip(np.rint(f / want_s), -127, 127).astype(np.int8)
+    assert np.array_equal(s.cpu().numpy(), want_s) and np.array_equal(q.cpu().numpy(), want_q)
+
+
 @pytest.mark.parametrize("n,H,Hkv,d,f16", [(1, 32, 8, 128, True), (300, 32, 8, 128, True), (4099, 32, 8, 128, False),
                                            (20000, 16, 2, 64, True), (32769, 32, 8, 128, True),
                                            (131072, 32, 8, 128, False), (131329, 32, 8, 128, False)])
@@ -185,6 +208,18 @@ def test_decode_bf16_matches_sdpa(dev):
     out = decode_bf16(q.to(dev), k.to(dev), v.to(dev), d ** -0.5)
     ref = oracle.sdpa_ref(q[:, None], k, v, causal=False, scale=d ** -0.5, groups=H // Hkv)[:, 0]
     _check(out, ref, "decode_bf16")
+
+
+@pytest.mark.parametrize("B,Hh,T,d", [(1, 40, 1, 128), (1, 7, 11000, 128), (2, 5, 20000, 64), (1, 33, 3000, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rope_head_groups_bitwise(B, Hh, T, d, dtype, dev):
+    """One and two heads per thread (an odd head count leaves a group short), bit for bit the host formula."""
+    print(f"case rope_head_groups {B} {Hh} {T} {d} {dtype}", flush=True)
+    cos, sin = rope_cos_sin(T, d, dtype=dtype)
+    x = _rand((B, Hh, T, d), 9, 2.0).to(dtype)
+    for y in (x.to(dev), x.to(dev).transpose(1, 2).contiguous().transpose(1, 2)):
+        rope_inplace(y, cos.to(dev), sin.to(dev))
+        assert torch.equal(y.cpu(), rope_host(x, cos, sin))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

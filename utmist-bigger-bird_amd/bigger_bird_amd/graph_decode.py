@@ -307,7 +307,7 @@ class StaticDecoder:
         for i, plan in enumerate(self.plans):
             layer = plan.layer
             hid, q, k, v, kv, qk = self._norm_qkv(plan, layer.input_layernorm, hid, pending)
-            if q.dtype == torch.bfloat16 and cos.dtype == torch.bfloat16:
+            if q.dtype in (torch.bfloat16, torch.float16) and cos.dtype == q.dtype:
                 if qk is not None:
                     rope_inplace(qk, cos, sin)
                 else:
