@@ -90,6 +90,18 @@ BB_DEV float slot_reduce_scatter(const float (&p)[G], int sub) {
   rs_round<G2, 0xB1>(v, (sub & 1) != 0);
   return v[0];
 }
+// Sum and maximum over the 8 key slots of a wave (lane bits 3..5), the same bits in every lane: row_ror 8, then the
+// permlane16 and permlane32 swaps, all inside the VALU (a __shfl_xor is an LDS crossbar round trip per value).
+BB_DEV float slots_sum(float v) {
+  v += dpp_mov<0x128>(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return xhalf_sum(__uint_as_float(a[0]) + __uint_as_float(a[1]));
+}
+BB_DEV float slots_max(float v) {
+  v = fmaxf(v, dpp_mov<0x128>(v));
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return xhalf_max(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+}
 constexpr int log2_heads(int g) { return g >= 8 ? 3 : g >= 4 ? 2 : g >= 2 ? 1 : 0; }
 BB_DEV u32x4_t ld16_nt(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)); }
 
@@ -133,8 +145,10 @@ BB_DEV void store_appended(const RowAppend& a, int kv, int64_t j, int sub, const
 // two keys per slot and step (their K and V rows in flight together). Route row r holds GR query heads (GR = groups
 // for pooled routes [Hkv, R], 1 for per-head routes [H, R]) and reads KV head (r GR) / groups. Virtual key
 // j < front -> position j; j < front + window -> n - window + (j - front); otherwise the routed index; positions
-// outside [0, n) are skipped (kernels/bigger_bird_decode.py:38-47). The key slots of a wave combine through lane
-// shuffles, the four waves through LDS. XS (the fused decode step after its routing pass): every key's score is
+// outside [0, n) are skipped (kernels/bigger_bird_decode.py:38-47). The key slots of a wave combine through lane moves
+// inside the VALU, the four waves through LDS (with three rounds of __shfl_xor, rescaling in each, a decode_step took 1.6
+// to 2 us more: 131072 keys routed 104.0 -> 102.2 us, 32768 keys dense 36.5 -> 34.7; four, six or eight keys per step
+// where the scores come from the routing pass: 102.9, 102.6 and 104.2). XS (the fused decode step after its routing pass): every key's score is
 // already in the routing workspace (p.xs, [H][xs_stride], log2 units, computed from the same q and K rows), so only
 // the V rows are read.
 constexpr int kSdThreads = 256;
@@ -142,6 +156,7 @@ constexpr float kSdRescale = 8.0f;
 
 template <int D, int GR, bool F16, bool XS>
 __global__ __launch_bounds__(kSdThreads) void sparse_decode_kernel(SparseDecodeParams p) {
+  constexpr int U = 2;  // keys per slot and step
   constexpr int LPK = kSlotLanes, DPL = D / LPK, KPW = 64 / LPK, SLOTS = kSdThreads / LPK, NW = kSdThreads / 64;
   __shared__ float part_m[NW][GR];
   __shared__ float part_l[NW][GR];
@@ -174,11 +189,11 @@ __global__ __launch_bounds__(kSdThreads) void sparse_decode_kernel(SparseDecodeP
   const int32_t* irow = p.idx + (int64_t)r * p.si0;
   const uint16_t* kbase = p.k + (int64_t)kv * p.sk0;
   const uint16_t* vbase = p.v + (int64_t)kv * p.sv0;
-  for (int64_t j0 = j_begin + slot; j0 < j_end; j0 += 2 * SLOTS) {
-    int64_t pos[2];
-    bool ok[2];
+  for (int64_t j0 = j_begin + slot; j0 < j_end; j0 += U * SLOTS) {
+    int64_t pos[U];
+    bool ok[U];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int64_t j = j0 + u * SLOTS;
       int64_t ps;
       if (j < p.front) ps = j;
@@ -187,10 +202,10 @@ __global__ __launch_bounds__(kSdThreads) void sparse_decode_kernel(SparseDecodeP
       ok[u] = j < j_end && ps >= 0 && ps < n;  // the 8 lanes of a key slot agree
       pos[u] = ok[u] ? ps : 0;
     }
-    u32x4_t kw[2][DPL / 8], vw[2][DPL / 8];
-    float xs[2][GR];  // XS: the keys' scores (log2 units) from the routing pass of the same step
+    u32x4_t kw[U][DPL / 8], vw[U][DPL / 8];
+    float xs[U][GR];  // XS: the keys' scores (log2 units) from the routing pass of the same step
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       const bool fresh = ok[u] && pos[u] == jnew;
       const uint16_t* ks = fresh ? p.app.knew + (int64_t)kv * p.app.skn : kbase + pos[u] * p.sk1;
       const uint16_t* vs = fresh ? p.app.vnew + (int64_t)kv * p.app.svn : vbase + pos[u] * p.sv1;
@@ -205,7 +220,7 @@ __global__ __launch_bounds__(kSdThreads) void sparse_decode_kernel(SparseDecodeP
       }
     }
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
       float s[GR];
       if constexpr (!XS) {
@@ -240,19 +255,15 @@ __global__ __launch_bounds__(kSdThreads) void sparse_decode_kernel(SparseDecodeP
       }
     }
   }
-  // combine the 8 key slots of the wave (lane bits 3..5), then the waves through LDS
+  // combine the 8 key slots of the wave, then the waves through LDS
 #pragma unroll
-  for (int off = LPK; off < 64; off <<= 1)
+  for (int h = 0; h < GR; ++h) {
+    const float mn = slots_max(m[h]), w = fast_exp2(m[h] - mn);
+    m[h] = mn;
+    l[h] = slots_sum(l[h] * w);
 #pragma unroll
-    for (int h = 0; h < GR; ++h) {
-      const float mo = __shfl_xor(m[h], off), lo = __shfl_xor(l[h], off);
-      const float mn = fmaxf(m[h], mo);
-      const float a = fast_exp2(m[h] - mn), b = fast_exp2(mo - mn);
-      m[h] = mn;
-      l[h] = l[h] * a + lo * b;
-#pragma unroll
-      for (int e = 0; e < DPL; ++e) acc[h][e] = acc[h][e] * a + __shfl_xor(acc[h][e], off) * b;
-    }
+    for (int e = 0; e < DPL; ++e) acc[h][e] = slots_sum(acc[h][e] * w);
+  }
   if (kslot == 0) {
 #pragma unroll
     for (int h = 0; h < GR; ++h) {
