@@ -11,6 +11,7 @@
 
 #include "bb_common.h"
 #include "bb_internal.h"
+#include "bb_slots.h"
 
 namespace bb {
 namespace {
@@ -138,19 +139,25 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const int8_t* __restric
 
 // ---------------------------------------------------------------------------------------------------------------
 // INT8 decode on the VALU (the shapes decode_mfma_kernel below is not built for). Workgroup (split s, KV head g): 4
-// waves; a wave walks keys 8 at a time, 8 lanes per key row (D / 8 values each).
+// waves, 8 lanes per key row (D / 8 values each), 32 key slots, U keys per slot and step with their K and V rows and
+// scales in flight together. K goes to packed bf16 pairs (exact for int8) and q . k runs on v_dot2c_f32_bf16; V is
+// converted once per key for all G heads. The 8 lanes of a slot, and at the end the 8 slots of a wave, combine on VALU lane
+// moves, the four waves through LDS. One key per slot and step, reduced through the LDS crossbar, left the loads' latency
+// exposed. Whole calls over 131072 keys at head_dim 128: 16 KV heads x 2 query heads 230 -> 163 us, 32 x 1 454 -> 314,
+// 4 x 8 164 -> 136 (16384 keys: 36 -> 29, 65 -> 46, 29 -> 27). Two or eight keys per step, plain instead of
+// non-temporal K / V loads: within 3%, 32 x 1 at 16384 keys 6% slower with plain loads.
 constexpr int kDecThreads = 256;
 constexpr float kDecRescale = 8.0f;
 
+BB_DEV uint32_t i8x2_to_bf16x2(uint32_t w, int hi) {  // bytes 2 hi, 2 hi + 1 of w
+  return pack_bf16x2((float)(int8_t)(w >> (16 * hi)), (float)(int8_t)(w >> (16 * hi + 8)));
+}
+
 template <int D, int G>
 __global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeParams p) {
-  constexpr int LPK = 8;             // lanes per key
-  constexpr int DPL = D / LPK;       // d values per lane
-  constexpr int KPW = 64 / LPK;      // keys per wave step
-  constexpr int SLOTS = kDecThreads / LPK;  // key slots per workgroup (32)
-  __shared__ float part_m[SLOTS][G];
-  __shared__ float part_l[SLOTS][G];
-  __shared__ float part_o[SLOTS][G][D];
+  constexpr int LPK = kSlotLanes, DPL = D / LPK, KPW = 64 / LPK, SLOTS = kDecThreads / LPK, NW = kDecThreads / 64;
+  constexpr int U = G >= 8 ? 2 : 4, W = DPL / 4;  // keys per slot and step; 32-bit words of a row per lane
+  __shared__ float part_m[NW][G], part_l[NW][G], part_o[NW][G][D];
 
   const int split = blockIdx.x, g = blockIdx.y;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -160,12 +167,12 @@ __global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeParams p) {
   int64_t j_end = j_begin + p.split_len;
   if (j_end > p.n) j_end = p.n;
 
-  float qv[G][DPL];
+  uint32_t qw[G][DPL / 2];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
     const uint16_t* qr = p.q + (int64_t)(g * G + h) * p.sq + DPL * sub;
 #pragma unroll
-    for (int e = 0; e < DPL; ++e) qv[h][e] = bf16_to_f32(qr[e]);
+    for (int e = 0; e < DPL / 2; ++e) qw[h][e] = (uint32_t)qr[2 * e] | ((uint32_t)qr[2 * e + 1] << 16);
   }
   float m[G], l[G], acc[G][DPL];
 #pragma unroll
@@ -175,78 +182,89 @@ __global__ __launch_bounds__(kDecThreads) void decode_kernel(DecodeParams p) {
 #pragma unroll
     for (int e = 0; e < DPL; ++e) acc[h][e] = 0.0f;
   }
-
-  for (int64_t j = j_begin + slot; j < j_end; j += SLOTS) {
-    float kf[DPL], vf[DPL];
-    const int64_t row = j * p.Hkv + g;
-    const int8_t* kr = p.k8 + row * D + DPL * sub;
-    const int8_t* vr = p.v8 + row * D + DPL * sub;
-    const float ks = load_scale(p.ks, row, p.scale_is_f16), vs = load_scale(p.vs, row, p.scale_is_f16);
-    // the lane's DPL bytes and no more: at head_dim 64 a 16-byte load would reach past the last row of the cache
-    uint32_t kw[DPL / 4], vw[DPL / 4];
+  // the lane's DPL bytes of a row and no more (at head_dim 64 a 16-byte load would reach past the last row of the
+  // cache); a slot's 8 lanes read the whole 128-byte row in one non-temporal instruction, or half a line plainly
+  auto load_row = [&](const int8_t* r, uint32_t (&w)[W]) {
     if constexpr (DPL == 16) {
-      const u32x4_t a = ld16(kr), b = ld16(vr);
+      const u32x4_t a = ld16_nt(r);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
+      for (int i = 0; i < 4; ++i) w[i] = a[i];
     } else {
       static_assert(DPL == 8, "8 or 16 bytes per lane");
-      const u32x2_t a = *reinterpret_cast<const u32x2_t*>(kr), b = *reinterpret_cast<const u32x2_t*>(vr);
+      const u32x2_t a = *reinterpret_cast<const u32x2_t*>(r);
+      w[0] = a[0];
+      w[1] = a[1];
+    }
+  };
+  for (int64_t j0 = j_begin + slot; j0 < j_end; j0 += U * SLOTS) {
+    uint32_t kw[U][W], vw[U][W];
+    float ks[U], vs[U];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) { kw[i] = a[i]; vw[i] = b[i]; }
+    for (int u = 0; u < U; ++u) {
+      const int64_t j = j0 + u * SLOTS < j_end ? j0 + u * SLOTS : j0;
+      const int64_t row = j * p.Hkv + g;
+      load_row(p.k8 + row * D + DPL * sub, kw[u]);
+      load_row(p.v8 + row * D + DPL * sub, vw[u]);
+      ks[u] = load_scale(p.ks, row, p.scale_is_f16);
+      vs[u] = load_scale(p.vs, row, p.scale_is_f16);
     }
 #pragma unroll
-    for (int e = 0; e < DPL; ++e) {
-      kf[e] = (float)(int8_t)((kw[e >> 2] >> (8 * (e & 3))) & 0xffu);
-      vf[e] = (float)(int8_t)((vw[e >> 2] >> (8 * (e & 3))) & 0xffu);
-    }
-    float s[G];
+    for (int u = 0; u < U; ++u) {
+      if (j0 + u * SLOTS >= j_end) break;  // the 8 lanes of a key slot agree
+      uint32_t kp[DPL / 2];
+      float vf[DPL];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float t = 0.0f;
+      for (int e = 0; e < DPL / 2; ++e) kp[e] = i8x2_to_bf16x2(kw[u][e >> 1], e & 1);
 #pragma unroll
-      for (int e = 0; e < DPL; ++e) t = fmaf(qv[h][e], kf[e], t);
-      s[h] = t;
-    }
+      for (int e = 0; e < DPL; ++e) vf[e] = (float)(int8_t)(vw[u][e >> 2] >> (8 * (e & 3)));
 #pragma unroll
-    for (int off = 1; off < LPK; off <<= 1)
+      for (int h = 0; h < G; ++h) {
+        float t = 0.0f;
 #pragma unroll
-      for (int h = 0; h < G; ++h) s[h] += __shfl_xor(s[h], off);
+        for (int e = 0; e < DPL / 2; ++e) t = dot2<false>(qw[h][e], kp[e], t);
+        const float x = slot_sum8(t) * ks[u] * p.c;
+        if (x > m[h] + kDecRescale) {
+          const float alpha = fast_exp2(m[h] - x);
+          m[h] = x;
+          l[h] *= alpha;
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float x = s[h] * ks * p.c;
-      if (x > m[h] + kDecRescale) {
-        const float alpha = fast_exp2(m[h] - x);
-        m[h] = x;
-        l[h] *= alpha;
+          for (int e = 0; e < DPL; ++e) acc[h][e] *= alpha;
+        }
+        const float pr = fast_exp2(x - m[h]);
+        l[h] += pr;
+        const float pv = pr * vs[u];
 #pragma unroll
-        for (int e = 0; e < DPL; ++e) acc[h][e] *= alpha;
+        for (int e = 0; e < DPL; ++e) acc[h][e] = fmaf(pv, vf[e], acc[h][e]);
       }
-      const float pr = fast_exp2(x - m[h]);
-      l[h] += pr;
-      const float pv = pr * vs;
-#pragma unroll
-      for (int e = 0; e < DPL; ++e) acc[h][e] = fmaf(pv, vf[e], acc[h][e]);
     }
   }
-  // workgroup combine of the SLOTS partial states per head
-  if (sub == 0) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) { part_m[slot][h] = m[h]; part_l[slot][h] = l[h]; }
+  for (int h = 0; h < G; ++h) {
+    const float mn = slots_max(m[h]), w = fast_exp2(m[h] - mn);
+    const float lt = slots_sum(l[h] * w);
+#pragma unroll
+    for (int e = 0; e < DPL; ++e) acc[h][e] = slots_sum(acc[h][e] * w);
+    if (lane == 0) {
+      part_m[wave][h] = mn;
+      part_l[wave][h] = lt;
+    }
+    if (kslot == 0) {
+#pragma unroll
+      for (int e = 0; e < DPL; ++e) part_o[wave][h][DPL * sub + e] = acc[h][e];
+    }
   }
-#pragma unroll
-  for (int h = 0; h < G; ++h)
-#pragma unroll
-    for (int e = 0; e < DPL; ++e) part_o[slot][h][DPL * sub + e] = acc[h][e];
   __syncthreads();
   for (int t = tid; t < G * D; t += kDecThreads) {
     const int h = t / D, d = t % D;
     float M = -1.0e30f;
-    for (int s2 = 0; s2 < SLOTS; ++s2) M = fmaxf(M, part_m[s2][h]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, part_m[w][h]);
     float L = 0.0f, O = 0.0f;
-    for (int s2 = 0; s2 < SLOTS; ++s2) {
-      const float w = fast_exp2(part_m[s2][h] - M);
-      L += w * part_l[s2][h];
-      O += w * part_o[s2][h][d];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float wt = fast_exp2(part_m[w][h] - M);
+      L += wt * part_l[w][h];
+      O += wt * part_o[w][h][d];
     }
     float* dst = p.part + ((int64_t)(g * G + h) * p.n_splits + split) * (D + 2);
     dst[d] = O;
