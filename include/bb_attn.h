@@ -267,6 +267,14 @@ size_t bb_topk_f32_workspace(int rows, int64_t n);
 int bb_argmax(const void* x, int64_t n, int dtype, int64_t* out, void* stream);
 
 /*
+ * bb_argmax into *token with the bookkeeping of a greedy decode step (modal_rd/graph_decode.py:201-205) in the same
+ * launch: tokens[*made] = the token when *made lies in [0, cap), then *made, *pos and *slot grow by one (all int64 in
+ * device memory).
+ */
+int bb_argmax_step(const void* x, int64_t n, int dtype, int64_t* token, int64_t* made, int64_t* pos, int64_t* slot,
+                   int64_t* tokens, int64_t cap, void* stream);
+
+/*
  * RMSNorm of `rows` rows of x (row stride sx elements, D contiguous 16-bit values, bf16 or fp16 by is_f16) with
  * weight w [D] into out (row stride so): the arithmetic of transformers' LlamaRMSNorm (fp32 mean of squares,
  * rsqrt(mean + eps), round to the model dtype, times the weight, round). One launch per call, for the decode step's
@@ -310,6 +318,15 @@ int bb_gemv(const void* w, int64_t sw, int N, int K, const void* x, int glu, int
  */
 int bb_gemv_norm(const void* w, int64_t sw, int N, int K, const void* x, const void* res, const void* norm_w,
                  float eps, int glu, int is_f16, void* sum, void* y, void* stream);
+
+/*
+ * bb_gemv_norm of a fused q / k / v projection (heads of D = 32, 64 or 128 rows) with RoPE on the rows below rope_rows
+ * (whole heads), in one launch: cos / sin [D] of the token's position, in the weight's type. Bit-identical to bb_gemv_norm
+ * followed by bb_rope_inplace.
+ */
+int bb_gemv_norm_rope(const void* w, int64_t sw, int N, int K, const void* x, const void* res, const void* norm_w,
+                      float eps, const void* cos, const void* sin, int D, int rope_rows, int is_f16, void* sum, void* y,
+                      void* stream);
 
 /*
  * In-place RoPE on x [B, Hh, T, D] (strides sx[3]) with cos/sin [B, T, D] (strides sc[2]; 0 to broadcast), with

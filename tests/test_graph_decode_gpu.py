@@ -292,3 +292,45 @@ def test_linear_vec_norm_is_norm_then_gemv(n, k, glu, with_res, dtype, dev):
         xn = rms_norm(x, nw, 1e-5)
         assert total is x
     assert torch.equal(y, linear_vec(xn, w, glu=glu))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,hk,d,k,with_res", [(32, 8, 128, 4096, True), (8, 2, 64, 512, False), (5, 5, 128, 520, True),
+                                                   (3, 1, 32, 64, False), (64, 8, 128, 8192, True)])
+def test_projection_with_rope_bitwise(heads, hk, d, k, with_res, dtype, dev):
+    """linear_vec_norm(rope=...) equals linear_vec_norm and then rope_inplace on the q and k heads, bit for bit."""
+    from bigger_bird_amd import rope_inplace
+    from bigger_bird_amd.decode import linear_vec_norm
+
+    print(f"case projection_with_rope {heads}/{hk} d={d} k={k} res={with_res} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(k + d)
+    rows = (heads + 2 * hk) * d
+    w = (torch.randn(rows, k, device=dev, generator=g) * k ** -0.5).to(dtype)
+    x, r = (torch.randn(1, 1, k, device=dev, generator=g).to(dtype) for _ in range(2))
+    nw = (1 + 0.1 * torch.randn(k, device=dev, generator=g)).to(dtype)
+    ang = torch.rand(1, 1, d, device=dev, generator=g) * 6.28
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+    res = r if with_res else None
+    total, y = linear_vec_norm(x, res, nw, 1e-5, w)
+    want = y.clone()
+    rope_inplace(want[0, 0, :(heads + hk) * d].view(1, heads + hk, 1, d), cos, sin)
+    got_total, got = linear_vec_norm(x, res, nw, 1e-5, w, rope=(cos, sin, (heads + hk) * d))
+    assert torch.equal(got, want) and torch.equal(got_total, total)
+
+
+@pytest.mark.parametrize("n", [7, 512, 32000, 128256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_argmax_step(n, dtype, dev):
+    """argmax with a step's bookkeeping: the token, its record (none past the buffer) and the three counters."""
+    from bigger_bird_amd.decode import argmax_step
+
+    print(f"case argmax_step n={n} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(n)
+    ctl, out = torch.tensor([9, 100, -1, 0, 9], device=dev), torch.full((3,), -5, device=dev)
+    want = []
+    for _ in range(5):
+        x = torch.randn(n, device=dev, generator=g).to(dtype)
+        argmax_step(x, ctl[2:3], ctl[3:4], ctl[1:2], ctl[4:5], out)
+        want.append(int(x.float().argmax()))
+        assert int(ctl[2]) == want[-1]
+    assert ctl.tolist() == [9, 105, want[-1], 5, 14] and out.tolist() == want[:3]

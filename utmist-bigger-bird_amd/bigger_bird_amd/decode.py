@@ -247,6 +247,20 @@ def argmax_index(x, out=None):
     return out
 
 
+def argmax_step(x, token, made, pos, slot, tokens):
+    """argmax_index(x, out=token) with a greedy step's bookkeeping in the same launch: tokens[made] = token (within
+    tokens), then made, pos and slot (int64 [1] GPU tensors) grow by one."""
+    if not x.is_cuda or x.ndim != 1 or x.dtype not in _ARGMAX_KIND:
+        raise ValueError("argmax_step needs a 1-D fp32/bf16/fp16 GPU tensor")
+    x = x if x.stride(0) == 1 else x.contiguous()
+    for t in (token, made, pos, slot, tokens):
+        if t.dtype != torch.int64 or not t.is_cuda or not t.is_contiguous():
+            raise ValueError("argmax_step: int64 GPU tensors")
+    _lib.check(_lib.lib().bb_argmax_step(_lib.ptr(x), x.shape[0], _ARGMAX_KIND[x.dtype], _lib.ptr(token), _lib.ptr(made),
+                                         _lib.ptr(pos), _lib.ptr(slot), _lib.ptr(tokens), tokens.numel(),
+                                         _lib.stream_of(x)))
+
+
 def _matrix16(x, d):
     """x as [rows, d] with 16-byte aligned rows (a copy only when x's layout does not allow it)."""
     x2 = x.reshape(-1, d)
@@ -333,17 +347,22 @@ def linear_vec(x, weight, glu=False):
     return y
 
 
-def linear_vec_norm(x, res, norm_weight, eps, weight, glu=False):
+def linear_vec_norm(x, res, norm_weight, eps, weight, glu=False, rope=None):
     """`linear_vec` on the RMSNorm of one hidden row, in one launch: returns (x + res, linear_vec(rms_norm(x + res)))
-    (res None: (x, linear_vec(rms_norm(x)))), bit-identical to add_rms_norm / rms_norm followed by linear_vec."""
+    (res None: (x, linear_vec(rms_norm(x)))), bit-identical to add_rms_norm / rms_norm followed by linear_vec.
+    rope = (cos, sin, rotated rows): weight is a fused q / k / v projection of heads of cos.numel() rows, and the heads
+    below that row leave rotated (bit-identical to rope_inplace on them)."""
     m, k = weight.shape
     if not gemv_ok(weight, x) or not x.is_cuda or k > 8192 or norm_weight.dtype != x.dtype:
         raise ValueError("linear_vec_norm needs a 16-bit GPU weight [N, K] (K % 8 == 0, K <= 8192, aligned rows), "
                          "an input and a norm weight of its dtype")
     if x.numel() != k or norm_weight.numel() != k or (res is not None and (res.numel() != k or res.dtype != x.dtype)):
         raise ValueError("linear_vec_norm takes one token: x, res and the norm weight must hold K values")
-    if glu and m % 2:
+    if glu and (m % 2 or rope is not None):
         raise ValueError("linear_vec_norm(glu=True) needs a [2N, K] gate / up weight")
+    if rope is not None and any(t.dtype != x.dtype or t.device != x.device or t.numel() != rope[0].numel()
+                                or not t.is_contiguous() for t in rope[:2]):
+        raise ValueError("linear_vec_norm: cos and sin must be contiguous rows of one head_dim in x's dtype")
     n = m // 2 if glu else m
 
     def flat(t):
@@ -354,6 +373,13 @@ def linear_vec_norm(x, res, norm_weight, eps, weight, glu=False):
     r1 = flat(res) if res is not None else None
     total = torch.empty_like(x) if res is not None else x
     y = torch.empty(x.shape[:-1] + (n,), dtype=x.dtype, device=x.device)
+    if rope is not None:
+        cos, sin, rows = rope
+        _lib.check(_lib.lib().bb_gemv_norm_rope(
+            _lib.ptr(weight), weight.stride(0), n, k, _lib.ptr(x1), _lib.ptr(r1), _lib.ptr(w1), float(eps), _lib.ptr(cos),
+            _lib.ptr(sin), cos.numel(), int(rows), int(x.dtype == torch.float16), _lib.ptr(total) if r1 is not None else None,
+            _lib.ptr(y), _lib.stream_of(x)))
+        return total, y
     _lib.check(_lib.lib().bb_gemv_norm(_lib.ptr(weight), weight.stride(0), n, k, _lib.ptr(x1),
                                        _lib.ptr(r1) if r1 is not None else None, _lib.ptr(w1), float(eps), int(glu),
                                        int(x.dtype == torch.float16), _lib.ptr(total) if r1 is not None else None,

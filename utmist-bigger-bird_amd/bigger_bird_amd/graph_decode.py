@@ -10,7 +10,7 @@ generate / EOS / rewind / feed protocol. The design is this package's own:
   and `load` copies the kept rows in.
 * State. A 5-slot int64 control block on the GPU holds (n, position, token, produced, slot): the filled cache rows,
   the RoPE position and id of the next input token, the number of tokens produced since `load`, and the cache row
-  the next token's K/V go to. A step advances the block with two vector adds, so every launch in it has a fixed
+  the next token's K/V go to. A step claims its row with one vector add and advances the block in the argmax launch, so every launch in it has a fixed
   shape and reads its varying values from device memory: the step is captured once and replayed per token.
 * Step (one token through the model): embedding; per layer RMSNorm -> one fused QKV projection (the q, k and v
   weights concatenated once at construction when they are plain bias-free Linear layers of one dtype) -> RoPE on q and
@@ -20,7 +20,8 @@ generate / EOS / rewind / feed protocol. The design is this package's own:
   by a one-workgroup HIP argmax written straight into the control block. The projections run as bb_gemv (one token:
   a matrix-vector product streaming the weight once, faster at batch 1 than the vendor GEMM) where the weight is a
   16-bit bias-free Linear with K <= 16384, and each residual add and RMSNorm rides in the launch of the projection
-  that follows it (bb_gemv_norm): 7 launches per Llama layer (q/k/v, RoPE, decode, merge, o, gate / up, down).
+  that follows it (bb_gemv_norm; the q/k/v one also rotates q and k, and the final norm rides in lm_head's): 6 launches
+  per Llama layer (q/k/v, decode, merge, o, gate / up, down).
 * Attention per layer: one bb_decode_step. Dense layers run split-K flash decoding over the filled rows (front 0,
   window = capacity, no routes, length read on the GPU); `sparse_decode={"front", "window", "routed"}` switches the
   non-dense RDAttention layers to fused decode routing (pooled per KV head) + sparse decode. The first kernel that
@@ -42,13 +43,13 @@ from transformers.cache_utils import DynamicLayer
 from transformers.models.llama.modeling_llama import apply_rotary_pos_emb
 
 from .attention import rope_inplace
-from .decode import (add_rms_norm, argmax_index, decode_step, gemv_ok, linear_vec, linear_vec_norm, rms_norm,
+from .decode import (add_rms_norm, argmax_step, decode_step, gemv_ok, linear_vec, linear_vec_norm, rms_norm,
                      silu_mul)
 
 # Control block: slot indices and the per-step / per-token increments.
 N, POS, TOK, MADE, SLOT = range(5)
 _CLAIM = (1, 0, 0, 0, 0)    # a step first grows the cache by the row it is about to write (at SLOT)
-_ADVANCE = (0, 1, 0, 1, 1)  # ... and ends one position further, with one more token produced and the next free row
+# (its end, one position further, with one more token produced and the next free row, rides in the argmax launch)
 _UNDO = (1, 1, 0, 1, 1)     # one consumed token taken back (rewind)
 
 
@@ -162,8 +163,7 @@ class StaticDecoder:
         with torch.inference_mode(False):
             self.arena = torch.zeros(len(layers), 2, self.hk, self.capacity, self.d, device=dev, dtype=dt)
             self.ctl = torch.zeros(5, dtype=torch.int64, device=dev)
-            self._claim, self._advance, self._undo = (torch.tensor(v, dtype=torch.int64, device=dev)
-                                                      for v in (_CLAIM, _ADVANCE, _UNDO))
+            self._claim, self._undo = (torch.tensor(v, dtype=torch.int64, device=dev) for v in (_CLAIM, _UNDO))
             self.out = torch.zeros(self.capacity, dtype=torch.int64, device=dev)
             self.no_routes = torch.empty(self.hk, 0, dtype=torch.int32, device=dev)
             # views made here, outside inference mode, so that later in-place updates are allowed in either mode
@@ -257,26 +257,32 @@ class StaticDecoder:
         o = o.reshape(1, 1, -1)
         return linear_vec(o, plan.base.o_proj.weight) if plan.o_vec else plan.base.o_proj(o)
 
-    def _norm_qkv(self, plan, module, hid, res):
+    def _norm_qkv(self, plan, module, hid, res, cos, sin):
         """The layer's input: hid + res (res None: hid), its norm and the q/k/v projections, as one bb_gemv_norm
         launch where the modules allow. Returns the new hid and q [1, H, 1, d], k and v [1, Hkv, 1, d], and, with the
-        fused projection, the [2, Hkv, 1, d] view of its K and V part (so RoPE on k in place also lands there) and the
-        [1, H + Hkv, 1, d] view of q and k together (one RoPE launch for both)."""
+        fused projection, the [2, Hkv, 1, d] view of its K and V part (so RoPE on k in place also lands there), the
+        [1, H + Hkv, 1, d] view of q and k together (one RoPE launch for both), and whether q and k already are
+        rotated (the projection's launch does it when cos / sin are plain rows of the model's dtype)."""
         h, hk, d = self.h, self.hk, self.d
         f = self._fast_norm(module, hid)
         if plan.qkv_vec and f and hid.shape[-1] <= 8192 and (res is None or res.dtype == hid.dtype):
-            hid, y = linear_vec_norm(hid, res, *f, plan.qkv_w)
-            y = y[0, 0]
+            rope = None
+            if (d in (32, 64, 128) and all(t.dtype == hid.dtype and t.numel() == d and t.is_contiguous()
+                                           for t in (cos, sin))):
+                rope = (cos, sin, (h + hk) * d)
+            hid, y = linear_vec_norm(hid, res, *f, plan.qkv_w, rope=rope)
+            y, rotated = y[0, 0], rope is not None
         else:
             hid, x = self._add_norm(module, hid, res)
+            rotated = False
             if plan.qkv_w is None:
                 q, k, v = (p(x)[0, 0] for p in (plan.base.q_proj, plan.base.k_proj, plan.base.v_proj))
-                return hid, q.view(1, h, 1, d), k.view(1, hk, 1, d), v.view(1, hk, 1, d), None, None
+                return hid, q.view(1, h, 1, d), k.view(1, hk, 1, d), v.view(1, hk, 1, d), None, None, False
             y = (linear_vec(x, plan.qkv_w) if plan.qkv_vec else torch.nn.functional.linear(x, plan.qkv_w))[0, 0]
         q, k, v = y.split((h * d, hk * d, hk * d))
         kv = y[h * d:].view(2, hk, 1, d)
         qk = y[:(h + hk) * d].view(1, h + hk, 1, d)
-        return hid, q.view(1, h, 1, d), k.view(1, hk, 1, d), v.view(1, hk, 1, d), kv, qk
+        return hid, q.view(1, h, 1, d), k.view(1, hk, 1, d), v.view(1, hk, 1, d), kv, qk, rotated
 
     def _norm_mlp(self, plan, module, hid, res):
         """hid + res, its norm and the MLP: returns the new hid and the MLP's output. With the HIP GEMVs the norm
@@ -306,8 +312,10 @@ class StaticDecoder:
         pending = None  # the last MLP's output, added to hid together with the next norm
         for i, plan in enumerate(self.plans):
             layer = plan.layer
-            hid, q, k, v, kv, qk = self._norm_qkv(plan, layer.input_layernorm, hid, pending)
-            if q.dtype in (torch.bfloat16, torch.float16) and cos.dtype == q.dtype:
+            hid, q, k, v, kv, qk, rotated = self._norm_qkv(plan, layer.input_layernorm, hid, pending, cos, sin)
+            if rotated:
+                pass
+            elif q.dtype in (torch.bfloat16, torch.float16) and cos.dtype == q.dtype:
                 if qk is not None:
                     rope_inplace(qk, cos, sin)
                 else:
@@ -320,11 +328,18 @@ class StaticDecoder:
                 kv = torch.stack((k[0], v[0]))
             o = self._attend(i, plan, q[0, :, 0], kv[0, :, 0], kv[1, :, 0])
             hid, pending = self._norm_mlp(plan, layer.post_attention_layernorm, hid, self._o_proj(plan, o))
-        hid, x = self._add_norm(self.core.norm, hid, pending)
-        self.logits = self.model.lm_head(x)[0, -1]
-        argmax_index(self.logits, out=self._token_flat)
-        self.out.index_copy_(0, self.step_i, self._token_flat)
-        self.ctl.add_(self._advance)
+        self.logits = self._head(hid, pending)
+        argmax_step(self.logits, self._token_flat, self.step_i, self.position, self.ctl[SLOT:SLOT + 1], self.out)
+
+    def _head(self, hid, res):
+        """lm_head on the final norm of hid + res (res None: hid) -> [vocab]; one bb_gemv_norm launch where the modules
+        allow."""
+        head, f = self.model.lm_head, self._fast_norm(self.core.norm, hid)
+        if (f and _plain_linear(head) and gemv_ok(head.weight, hid) and hid.shape[-1] <= 8192
+                and (res is None or (res.dtype == hid.dtype and res.numel() == hid.numel()))):
+            return linear_vec_norm(hid, res, *f, head.weight)[1][0, -1]
+        _, x = self._add_norm(self.core.norm, hid, res)
+        return head(x)[0, -1]
 
     # ---- graph capture and running ----
     def capture(self):

@@ -830,7 +830,7 @@ int bb_gemv(const void* w, int64_t sw, int N, int K, const void* x, int glu, int
   if (!aligned(w, 16) || !aligned(x, 16) || sw % 8 || sw < K || !aligned(y, 2))
     return fail("gemv: W rows and x must be 16-byte aligned");
   return hip_status(bb::launch_gemv(static_cast<const uint16_t*>(w), sw, N, K, static_cast<const uint16_t*>(x), nullptr,
-                                    glu != 0, is_f16 ? 1 : 0, static_cast<uint16_t*>(y),
+                                    nullptr, glu != 0, is_f16 ? 1 : 0, static_cast<uint16_t*>(y),
                                     static_cast<hipStream_t>(stream)),
                     "bb_gemv");
 }
@@ -847,7 +847,7 @@ int bb_gemv_norm(const void* w, int64_t sw, int N, int K, const void* x, const v
   const bb::GemvNorm nm{static_cast<const uint16_t*>(res), static_cast<const uint16_t*>(norm_w), eps,
                         static_cast<uint16_t*>(sum)};
   return hip_status(bb::launch_gemv(static_cast<const uint16_t*>(w), sw, N, K, static_cast<const uint16_t*>(x), &nm,
-                                    glu != 0, is_f16 ? 1 : 0, static_cast<uint16_t*>(y),
+                                    nullptr, glu != 0, is_f16 ? 1 : 0, static_cast<uint16_t*>(y),
                                     static_cast<hipStream_t>(stream)),
                     "bb_gemv_norm");
 }
@@ -862,12 +862,44 @@ int bb_silu_mul(const void* g, const void* u, int64_t n, int is_f16, void* out, 
                     "bb_silu_mul");
 }
 
+int bb_gemv_norm_rope(const void* w, int64_t sw, int N, int K, const void* x, const void* res, const void* norm_w,
+                      float eps, const void* cos, const void* sin, int D, int rope_rows, int is_f16, void* sum, void* y,
+                      void* stream) {
+  g_err[0] = 0;
+  if (!w || !x || !norm_w || !y || !cos || !sin || (res != nullptr) != (sum != nullptr))
+    return fail("gemv_norm_rope: null argument");
+  if (N < 0 || K <= 0 || K % 8 || K > 8192)
+    return fail("gemv_norm_rope: K = %d must be a positive multiple of 8, at most 8192", K);
+  if ((D != 32 && D != 64 && D != 128) || N % D || rope_rows < 0 || rope_rows > N || rope_rows % D)
+    return fail("gemv_norm_rope: N and the rotated rows must be whole heads of 32, 64 or 128 rows");
+  if (!aligned(w, 16) || !aligned(x, 16) || !aligned(norm_w, 16) || (res && (!aligned(res, 16) || !aligned(sum, 16))) ||
+      sw % 8 || sw < K || !aligned(y, 2) || !aligned(cos, 2) || !aligned(sin, 2))
+    return fail("gemv_norm_rope: W rows, x, res, sum and the norm weight must be 16-byte aligned");
+  const bb::GemvNorm nm{static_cast<const uint16_t*>(res), static_cast<const uint16_t*>(norm_w), eps,
+                        static_cast<uint16_t*>(sum)};
+  const bb::GemvRope rp{static_cast<const uint16_t*>(cos), static_cast<const uint16_t*>(sin),
+                        D == 128 ? 6 : (D == 64 ? 5 : 4), rope_rows};
+  return hip_status(bb::launch_gemv(static_cast<const uint16_t*>(w), sw, N, K, static_cast<const uint16_t*>(x), &nm, &rp,
+                                    false, is_f16 ? 1 : 0, static_cast<uint16_t*>(y), static_cast<hipStream_t>(stream)),
+                    "bb_gemv_norm_rope");
+}
+int bb_argmax_step(const void* x, int64_t n, int dtype, int64_t* token, int64_t* made, int64_t* pos, int64_t* slot,
+                   int64_t* tokens, int64_t cap, void* stream) {
+  g_err[0] = 0;
+  if (!x || !token || !made || !pos || !slot || !tokens) return fail("argmax_step: null argument");
+  if (n <= 0 || n > 0x7ffffffe) return fail("argmax_step: row length %lld out of range", (long long)n);
+  if (dtype < 0 || dtype > 2) return fail("argmax_step: dtype must be 0 (fp32), 1 (bf16) or 2 (fp16)");
+  return hip_status(bb::launch_argmax(x, n, dtype, aligned(x, 16), token, bb::ArgmaxStep{made, pos, slot, tokens, cap},
+                                      static_cast<hipStream_t>(stream)),
+                    "bb_argmax_step");
+}
 int bb_argmax(const void* x, int64_t n, int dtype, int64_t* out, void* stream) {
   g_err[0] = 0;
   if (!x || !out) return fail("argmax: null argument");
   if (n <= 0 || n > 0x7ffffffe) return fail("argmax: row length %lld out of range", (long long)n);
   if (dtype < 0 || dtype > 2) return fail("argmax: dtype must be 0 (fp32), 1 (bf16) or 2 (fp16)");
-  return hip_status(bb::launch_argmax(x, n, dtype, aligned(x, 16), out, static_cast<hipStream_t>(stream)), "bb_argmax");
+  return hip_status(bb::launch_argmax(x, n, dtype, aligned(x, 16), out, bb::ArgmaxStep{},
+                                      static_cast<hipStream_t>(stream)), "bb_argmax");
 }
 
 int bb_stream_read(const void* buf, size_t bytes, uint32_t* sink, int workgroups, void* stream) {

@@ -61,6 +61,14 @@ BB_DEV float slot_reduce_scatter(const float (&p)[G], int sub) {
 }
 constexpr int log2_heads(int g) { return g >= 8 ? 3 : g >= 4 ? 2 : g >= 2 ? 1 : 0; }
 
+// x rounded to the element type and back, opaque to the compiler (which would otherwise fuse an fp16 product and add).
+template <bool F16>
+BB_DEV float round_elem(float x) {
+  uint32_t h = f32_to_elem<F16>(x);
+  asm volatile("" : "+v"(h));
+  return elem_to_f32<F16>((uint16_t)h);
+}
+
 // q row of one lane's pieces as packed pairs (DPL 16-bit values, DPL / 2 words).
 template <int DPL>
 BB_DEV void load_q_pairs(const uint16_t* qrow, int sub, uint32_t (&qw)[DPL / 2]) {
@@ -527,9 +535,11 @@ BB_DEV bool am_better(float a, int ia, float b, int ib) {
   return ia < ib;
 }
 
+// With `step` set the same thread also does the bookkeeping of a decode step (StaticDecoder's control block): the token
+// is recorded and the position, token count and write slot advance, which were two more launches of 3-5 us.
 template <typename T, int EPU>  // element type (float, bf16 / fp16 bits), elements per load
 __global__ __launch_bounds__(kAmThreads) void argmax_kernel(const T* __restrict__ x, int64_t n, int kind,
-                                                            int64_t* __restrict__ out) {
+                                                            int64_t* __restrict__ out, ArgmaxStep step) {
   __shared__ float wv[kAmThreads / 64];
   __shared__ int wi[kAmThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -540,21 +550,31 @@ __global__ __launch_bounds__(kAmThreads) void argmax_kernel(const T* __restrict_
   float bv = -__builtin_huge_valf();
   int bi = 0x7fffffff;
   const int64_t units = n / EPU;
-  for (int64_t u = tid; u < units; u += kAmThreads) {
-    T e[EPU];
-    if constexpr (EPU > 1) {
-      const u32x4_t w = *reinterpret_cast<const u32x4_t*>(x + u * EPU);
-      __builtin_memcpy(e, &w, sizeof(w));
-    } else {
-      e[0] = x[u];
+  constexpr int UF = 4;  // loads in flight per thread
+  for (int64_t u0 = tid; u0 < units; u0 += UF * kAmThreads) {
+    T e[UF][EPU];
+#pragma unroll
+    for (int f = 0; f < UF; ++f) {
+      const int64_t u = u0 + f * kAmThreads < units ? u0 + f * kAmThreads : u0;
+      if constexpr (EPU > 1) {
+        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(x + u * EPU);
+        __builtin_memcpy(e[f], &w, sizeof(w));
+      } else {
+        e[f][0] = x[u];
+      }
     }
 #pragma unroll
-    for (int k = 0; k < EPU; ++k) {
-      const float v = value(e[k]);
-      const int i = (int)(u * EPU + k);
-      if (am_better(v, i, bv, bi)) {
-        bv = v;
-        bi = i;
+    for (int f = 0; f < UF; ++f) {
+      const int64_t u = u0 + f * kAmThreads;
+      if (u >= units) break;
+#pragma unroll
+      for (int k = 0; k < EPU; ++k) {
+        const float v = value(e[f][k]);
+        const int i = (int)(u * EPU + k);
+        if (am_better(v, i, bv, bi)) {
+          bv = v;
+          bi = i;
+        }
       }
     }
   }
@@ -585,7 +605,15 @@ __global__ __launch_bounds__(kAmThreads) void argmax_kernel(const T* __restrict_
         bv = wv[w];
         bi = wi[w];
       }
-    out[0] = bi == 0x7fffffff ? 0 : bi;
+    const int64_t token = bi == 0x7fffffff ? 0 : bi;
+    out[0] = token;
+    if (step.made) {
+      const int64_t made = *step.made;
+      if (made >= 0 && made < step.cap) step.tokens[made] = token;
+      *step.made = made + 1;
+      *step.pos += 1;
+      *step.slot += 1;
+    }
   }
 }
 
@@ -716,10 +744,14 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // round(round(silu(g)) u) of the rounded g and u (silu_mul_kernel's arithmetic): the MLP's activation input.
 constexpr int kGvWaves = 4;
 constexpr int kGvMaxK = 16384;  // x staged in 32 KB of LDS
-template <bool F16, bool GLU, bool NORM, bool RES, int R, int A, int KS>
+// ROPE: W is a fused q / k / v projection of heads of 2^(rp.shift + 1) rows; a wave group's two rows are i and i + D / 2
+// of one head, so it holds both halves of a RoPE pair and writes rope_kernel's arithmetic on the rounded products for the
+// heads below row rp.rows (the separate RoPE launch took 4.5 us per layer).
+template <bool F16, bool GLU, bool NORM, bool RES, bool ROPE, int R, int A, int KS>
 __global__ __launch_bounds__(64 * kGvWaves) void gemv_kernel(const uint16_t* __restrict__ w, int64_t sw, int N, int K,
-                                                              const uint16_t* __restrict__ x, GemvNorm nm,
+                                                              const uint16_t* __restrict__ x, GemvNorm nm, GemvRope rp,
                                                               uint16_t* __restrict__ y, int rounds) {
+  static_assert(!ROPE || (R == 2 && !GLU), "a RoPE pair is a wave group's two rows");
   static_assert(!GLU || R % 2 == 0, "GLU rows come in (gate, up) pairs");
   static_assert(kGvWaves % KS == 0, "K parts split the workgroup's waves evenly");
   static_assert(!NORM || 64 * kGvWaves == kRnThreads, "the norm prologue runs on rms_norm_kernel's thread layout");
@@ -738,6 +770,10 @@ __global__ __launch_bounds__(64 * kGvWaves) void gemv_kernel(const uint16_t* __r
   // row r of round k: output group gid + k ngroups (rows past the end read the last row; their outputs are not
   // stored)
   auto row = [&](int k, int r) -> const uint16_t* {
+    if constexpr (ROPE) {  // pair pi: rows i and i + D / 2 of head pi / (D / 2)
+      const int pi = gid + k * ngroups < N / 2 ? gid + k * ngroups : N / 2 - 1, half = 1 << rp.shift;
+      return w + (int64_t)(((pi >> rp.shift) << (rp.shift + 1)) + (pi & (half - 1)) + r * half) * sw;
+    }
     const int o = (gid + k * ngroups) * OUTS + (GLU ? r / 2 : r);
     const int oc = o < N ? o : N - 1;
     return w + (int64_t)(GLU ? oc + (r & 1) * N : oc) * sw;
@@ -797,7 +833,20 @@ __global__ __launch_bounds__(64 * kGvWaves) void gemv_kernel(const uint16_t* __r
             }
           }
           const int out0 = (gid + ck * ngroups) * OUTS;
-          if (kp == 0 && lane < OUTS && out0 + lane < N) {
+          if constexpr (ROPE) {
+            const int pi = gid + ck * ngroups, half = 1 << rp.shift, i = pi & (half - 1);
+            const int row0 = ((pi >> rp.shift) << (rp.shift + 1)) + i;
+            if (kp == 0 && lane < 2 && pi < N / 2) {
+              const float a1 = round_elem<F16>(acc[0]), a2 = round_elem<F16>(acc[1]);
+              float v = lane ? a2 : a1;
+              if (row0 < rp.rows) {
+                const int d = i + lane * half;
+                const float c = elem_to_f32<F16>(rp.cos[d]), sn = elem_to_f32<F16>(rp.sin[d]);
+                v = round_elem<F16>(v * c) + round_elem<F16>((lane ? a1 : -a2) * sn);
+              }
+              y[row0 + lane * half] = f32_to_elem<F16>(v);
+            }
+          } else if (kp == 0 && lane < OUTS && out0 + lane < N) {
             float v = acc[0];  // acc[lane] with a static index
 #pragma unroll
             for (int r = 1; r < OUTS; ++r) v = lane == r ? acc[GLU ? 2 * r : r] : v;
@@ -890,21 +939,22 @@ hipError_t launch_kv_append(uint16_t* k, int64_t sk0, int64_t sk1, uint16_t* v, 
   return hipGetLastError();
 }
 
-hipError_t launch_argmax(const void* x, int64_t n, int kind, bool vec16, int64_t* out, hipStream_t stream) {
+hipError_t launch_argmax(const void* x, int64_t n, int kind, bool vec16, int64_t* out, const ArgmaxStep& step,
+                         hipStream_t stream) {
   if (n <= 0 || n > 0x7ffffffe) return hipErrorInvalidValue;
   if (kind == 0) {
     if (vec16)
       hipLaunchKernelGGL((argmax_kernel<uint32_t, 4>), dim3(1), dim3(kAmThreads), 0, stream,
-                         static_cast<const uint32_t*>(x), n, kind, out);
+                         static_cast<const uint32_t*>(x), n, kind, out, step);
     else
       hipLaunchKernelGGL((argmax_kernel<uint32_t, 1>), dim3(1), dim3(kAmThreads), 0, stream,
-                         static_cast<const uint32_t*>(x), n, kind, out);
+                         static_cast<const uint32_t*>(x), n, kind, out, step);
   } else if (vec16) {
     hipLaunchKernelGGL((argmax_kernel<uint16_t, 8>), dim3(1), dim3(kAmThreads), 0, stream,
-                       static_cast<const uint16_t*>(x), n, kind, out);
+                       static_cast<const uint16_t*>(x), n, kind, out, step);
   } else {
     hipLaunchKernelGGL((argmax_kernel<uint16_t, 1>), dim3(1), dim3(kAmThreads), 0, stream,
-                       static_cast<const uint16_t*>(x), n, kind, out);
+                       static_cast<const uint16_t*>(x), n, kind, out, step);
   }
   return hipGetLastError();
 }
@@ -939,38 +989,41 @@ hipError_t launch_rms_norm(const uint16_t* x, int64_t sx, const uint16_t* res, i
 constexpr int kGvR = 2, kGvA = 8, kGvKS = 2;
 constexpr int kGvMaxGroups = 1024;
 
-template <bool F16, bool GLU, bool NORM, bool RES>
+template <bool F16, bool GLU, bool NORM, bool RES, bool ROPE>
 hipError_t launch_gemv_t(const uint16_t* w, int64_t sw, int N, int K, const uint16_t* x, const GemvNorm& nm,
-                         uint16_t* y, hipStream_t stream) {
+                         const GemvRope& rp, uint16_t* y, hipStream_t stream) {
   // workgroups: at most kGvMaxGroups; each wave group takes `rounds` output groups, spread so that the last round
   // is as full as the others
   constexpr int outs = kGvWaves / kGvKS * (GLU ? kGvR / 2 : kGvR);  // outputs per workgroup and round
   const int64_t wg_needed = (N + outs - 1) / outs;
-  int cap = kGvMaxGroups;
-  if (const char* e = getenv("BB_GEMV_CAP")) cap = atoi(e);
-  const int rounds = (int)((wg_needed + cap - 1) / cap);
+  const int rounds = (int)((wg_needed + kGvMaxGroups - 1) / kGvMaxGroups);
   const unsigned grid = (unsigned)((wg_needed + rounds - 1) / rounds);
-  hipLaunchKernelGGL((gemv_kernel<F16, GLU, NORM, RES, kGvR, kGvA, kGvKS>), dim3(grid), dim3(64 * kGvWaves), 0,
-                     stream, w, sw, N, K, x, nm, y, rounds);
+  hipLaunchKernelGGL((gemv_kernel<F16, GLU, NORM, RES, ROPE, kGvR, kGvA, kGvKS>), dim3(grid), dim3(64 * kGvWaves), 0,
+                     stream, w, sw, N, K, x, nm, rp, y, rounds);
   return hipGetLastError();
 }
 
 template <bool F16, bool GLU>
 hipError_t launch_gemv_g(const uint16_t* w, int64_t sw, int N, int K, const uint16_t* x, const GemvNorm* nm,
-                         uint16_t* y, hipStream_t stream) {
-  if (!nm) return launch_gemv_t<F16, GLU, false, false>(w, sw, N, K, x, GemvNorm{}, y, stream);
-  if (nm->res) return launch_gemv_t<F16, GLU, true, true>(w, sw, N, K, x, *nm, y, stream);
-  return launch_gemv_t<F16, GLU, true, false>(w, sw, N, K, x, *nm, y, stream);
+                         const GemvRope* rp, uint16_t* y, hipStream_t stream) {
+  const GemvRope none{};
+  if (!nm) return launch_gemv_t<F16, GLU, false, false, false>(w, sw, N, K, x, GemvNorm{}, none, y, stream);
+  if constexpr (!GLU) {
+    if (rp && nm->res) return launch_gemv_t<F16, GLU, true, true, true>(w, sw, N, K, x, *nm, *rp, y, stream);
+    if (rp) return launch_gemv_t<F16, GLU, true, false, true>(w, sw, N, K, x, *nm, *rp, y, stream);
+  }
+  if (nm->res) return launch_gemv_t<F16, GLU, true, true, false>(w, sw, N, K, x, *nm, none, y, stream);
+  return launch_gemv_t<F16, GLU, true, false, false>(w, sw, N, K, x, *nm, none, y, stream);
 }
 
-hipError_t launch_gemv(const uint16_t* w, int64_t sw, int N, int K, const uint16_t* x, const GemvNorm* nm, bool glu,
-                       int f16, uint16_t* y, hipStream_t stream) {
+hipError_t launch_gemv(const uint16_t* w, int64_t sw, int N, int K, const uint16_t* x, const GemvNorm* nm,
+                       const GemvRope* rp, bool glu, int f16, uint16_t* y, hipStream_t stream) {
   if (N <= 0) return hipSuccess;
-  if (K <= 0 || K % 8 || K > kGvMaxK || (nm && K > kRnMaxD)) return hipErrorInvalidValue;
-  if (f16) return glu ? launch_gemv_g<true, true>(w, sw, N, K, x, nm, y, stream)
-                      : launch_gemv_g<true, false>(w, sw, N, K, x, nm, y, stream);
-  return glu ? launch_gemv_g<false, true>(w, sw, N, K, x, nm, y, stream)
-             : launch_gemv_g<false, false>(w, sw, N, K, x, nm, y, stream);
+  if (K <= 0 || K % 8 || K > kGvMaxK || (nm && K > kRnMaxD) || (rp && (!nm || glu))) return hipErrorInvalidValue;
+  if (f16) return glu ? launch_gemv_g<true, true>(w, sw, N, K, x, nm, rp, y, stream)
+                      : launch_gemv_g<true, false>(w, sw, N, K, x, nm, rp, y, stream);
+  return glu ? launch_gemv_g<false, true>(w, sw, N, K, x, nm, rp, y, stream)
+             : launch_gemv_g<false, false>(w, sw, N, K, x, nm, rp, y, stream);
 }
 
 hipError_t launch_silu_mul(const uint16_t* g, const uint16_t* u, int64_t n, int f16, uint16_t* out,

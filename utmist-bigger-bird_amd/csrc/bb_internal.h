@@ -184,10 +184,17 @@ struct GemvNorm {
   float eps;
   uint16_t* sum;        // x + res [K] (with res; must not overlap x or res)
 };
+// RoPE on the outputs of a fused q / k / v projection: heads of 2 << shift rows, the ones below `rows` rotated.
+struct GemvRope {
+  const uint16_t* cos;  // [D] of the token's position
+  const uint16_t* sin;
+  int shift, rows;
+};
 // y[N] = W[N, K] x[K] for one token (16-bit, row stride sw; K % 8 == 0, K <= 16384; 16-byte aligned rows and x);
-// nm: x replaced by its RMSNorm (K <= 8192); glu: W has 2N rows (gate over up) and y = round(round(silu(g)) u).
-hipError_t launch_gemv(const uint16_t* w, int64_t sw, int N, int K, const uint16_t* x, const GemvNorm* nm, bool glu,
-                       int f16, uint16_t* y, hipStream_t stream);
+// nm: x replaced by its RMSNorm (K <= 8192); rp (with nm, without glu; N a multiple of the head size): RoPE on y; glu: W
+// has 2N rows (gate over up) and y = round(round(silu(g)) u).
+hipError_t launch_gemv(const uint16_t* w, int64_t sw, int N, int K, const uint16_t* x, const GemvNorm* nm,
+                       const GemvRope* rp, bool glu, int f16, uint16_t* y, hipStream_t stream);
 // out = round(round(silu(g)) u) over n values (n % 8 == 0, 16-byte aligned).
 hipError_t launch_silu_mul(const uint16_t* g, const uint16_t* u, int64_t n, int f16, uint16_t* out,
                            hipStream_t stream);
@@ -196,7 +203,14 @@ hipError_t launch_silu_mul(const uint16_t* g, const uint16_t* u, int64_t n, int 
 hipError_t launch_kv_append(uint16_t* k, int64_t sk0, int64_t sk1, uint16_t* v, int64_t sv0, int64_t sv1,
                             const uint16_t* knew, int64_t skn, const uint16_t* vnew, int64_t svn, int heads, int D,
                             int64_t cap, int64_t* n_dev, int64_t n_inc, hipStream_t stream);
-hipError_t launch_argmax(const void* x, int64_t n, int kind, bool vec16, int64_t* out, hipStream_t stream);
+// The bookkeeping of a greedy step done with the argmax (made = null: none): tokens[*made] = the token (when *made lies
+// in [0, cap)), then *made, *pos and *slot grow by one.
+struct ArgmaxStep {
+  int64_t *made, *pos, *slot, *tokens;
+  int64_t cap;
+};
+hipError_t launch_argmax(const void* x, int64_t n, int kind, bool vec16, int64_t* out, const ArgmaxStep& step,
+                         hipStream_t stream);
 hipError_t launch_f32_keys(const float* vals, int64_t sv0, int rows, int64_t n, uint64_t* keys, hipStream_t stream);
 
 // RoPE in place (HF apply_rotary_pos_emb arithmetic in bf16, or fp16 when f16).
