@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void scores_kernel(RoutesParams p, RouteGeom g
 #pragma unroll
       for (int b = 0; b < 4; ++b) acc[a][b] = 0.0f;
     if constexpr (F16) {
-#pragma unroll 2
+#pragma unroll 8  // LDS reads further ahead of the FMAs: 2 to 8% against 2 (135.9 -> 125.5 us at 20011 tokens, head_dim 64)
       for (int dd = 0; dd < D; ++dd) {
         const u32x4_t qv = *reinterpret_cast<const u32x4_t*>(&qs[dd][8 * rg]);
         const u32x2_t kv = *reinterpret_cast<const u32x2_t*>(&ks[dd][4 * kg]);
