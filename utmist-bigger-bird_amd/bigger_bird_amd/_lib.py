@@ -102,16 +102,26 @@ def check(rc: int) -> None:
     raise RuntimeError(msg)
 
 
+# A one-token call is two launches of a few microseconds, so the lookups around them count: the stream handle without a
+# Stream object (2 us), pointers as plain integers (every argtype is declared) and array types made once.
+_I64S = tuple(ctypes.c_int64 * n for n in range(9))
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def i64s(*vals):
-    return (ctypes.c_int64 * len(vals))(*[int(v) for v in vals])
+    return (_I64S[len(vals)] if len(vals) < len(_I64S) else ctypes.c_int64 * len(vals))(*vals)
 
 
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream's handle on t's device, as an integer."""
+    device = t.get_device()  # -1 for a tensor that is not on a GPU: torch refuses it below
+    if _raw_stream is not None and device >= 0:
+        return _raw_stream(device)
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def require_gpu(*tensors, what="bigger_bird_amd"):
