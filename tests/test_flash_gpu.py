@@ -159,6 +159,23 @@ def test_split_chunks(t, n, front, window, noncausal, heads, d, dev):
     _check(out, ref, "split_chunks")
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float16, 64)])
+def test_split_chunks_infinite_value(dtype, d, dev):
+    """An infinite value in the first key chunk reaches its column as infinity and leaves the others alone: the merge
+    weights no row that is not a chunk's own."""
+    print(f"case split_infinite {dtype} d={d}", flush=True)
+    from bigger_bird_amd import exact_attention
+
+    q, k, v = _rand((8, 5, d), 44, dtype), _rand((2, 1500, d), 45, dtype), _rand((2, 1500, d), 46, dtype)
+    kw = dict(num_heads=8, kv_groups=4, scale=d ** -0.5)
+    want = exact_attention(q.to(dev), k.to(dev), v.to(dev), **kw)
+    v[:, 3, 7] = float("inf")
+    got = exact_attention(q.to(dev), k.to(dev), v.to(dev), **kw)
+    assert torch.isposinf(got[..., 7]).all()
+    keep = torch.arange(d, device=dev) != 7
+    assert torch.equal(got[..., keep], want[..., keep])
+
+
 def test_full_budget_equals_dense_causal(dev):
     """modal_rd/selfcheck.py:36-41: routing every column outside sink/window gives exact causal attention."""
     print("case full_budget", flush=True)

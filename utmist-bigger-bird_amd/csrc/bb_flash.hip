@@ -405,7 +405,8 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashParams p) {
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const float wc = live[u] ? __shfl(w, (c + u) & 63) : 0.0f;
+        if (!live[u]) continue;  // uniform; a weight of zero would turn an infinite value of the stand-in row into NaN
+        const float wc = __shfl(w, (c + u) & 63);
 #pragma unroll
         for (int i = 0; i < PER; ++i) acc[i] += wc * v[u][i];
       }
