@@ -201,6 +201,23 @@ def test_one_token_over_16bit_cache(n, H, Hkv, d, layout, dtype, dev):
     _check(out, ref, f"one_token n={n}")
 
 
+@pytest.mark.parametrize("k_shape,v_shape", [((8, 300, 128), (8, 200, 128)), ((16, 300, 128), (16, 300, 128)),
+                                             ((8, 300, 64), (8, 300, 64))])
+def test_one_token_refuses_mismatched_cache(k_shape, v_shape, dev):
+    """An fp16 token over K and V of different lengths, head counts or widths is an error, as for several tokens."""
+    from types import SimpleNamespace
+
+    from bigger_bird_amd import RDAttention
+
+    print(f"case one_token_refused {k_shape} {v_shape}", flush=True)
+    base = SimpleNamespace(config=SimpleNamespace(num_attention_heads=32, num_key_value_heads=8), layer_idx=0, head_dim=128,
+                           scaling=0.1, q_proj=None, k_proj=None, v_proj=None, o_proj=None)
+    q = torch.zeros(1, 32, 1, 128, dtype=torch.float16, device=dev)
+    k, v = (torch.zeros(1, *s, dtype=torch.float16, device=dev) for s in (k_shape, v_shape))
+    with pytest.raises(ValueError, match="matching heads and dimensions"):
+        RDAttention(base).exact_attention(q, k, v, 1, k.shape[2])
+
+
 def test_decode_bf16_matches_sdpa(dev):
     print("case decode_bf16", flush=True)
     n, H, Hkv, d = 5000, 32, 8, 128

@@ -214,7 +214,8 @@ class RDAttention(nn.Module):
             if q.dtype == torch.bfloat16:
                 from .kv_int8 import decode_bf16
                 return decode_bf16(q[0, :, 0], k[0], v[0], self.scaling)[None, :, None]
-            if q.dtype == torch.float16 and k.dtype == q.dtype and v.dtype == q.dtype:
+            if (q.is_cuda and q.dtype == torch.float16 and k.dtype == q.dtype and v.dtype == q.dtype and k.shape == v.shape
+                    and q.shape[1] == k.shape[1] * self.groups and q.shape[-1] == k.shape[-1] == self.head_dim):
                 # the prefill kernels took this before: a V^T pass over the whole cache and one live row of 64 in
                 # every tile (4099 rows of 8 KV heads: 26 us a call against 15, 131072 rows 226 us against 91)
                 return decode_dense(q[0, :, 0], k[0], v[0], self.scaling)[None, :, None]

@@ -74,6 +74,8 @@ def decode_dense(q, k, v, scale):
     all keys in the window and no routes (fp32 probabilities; split over the chip and merged, two launches)."""
     h, d = q.shape
     hk, n, _ = k.shape
+    if k.shape != v.shape or k.shape[-1] != d or h % hk:
+        raise ValueError("q [H,D] and k/v [Hkv,N,D] must match")
     _lib.require_gpu(q, k, v, what="decode_dense")
     k, v = _rows16(k), _rows16(v)
     q = q if q.stride(-1) == 1 else q.contiguous()
