@@ -109,6 +109,34 @@ def test_graph_matches_model_forward(arm, extra, dev):
             tok = nxt  # teacher forcing with the graph's token
 
 
+@pytest.mark.parametrize("how", ["hook", "forward", "subclass"])
+def test_customised_lm_head_is_called(how, dev):
+    """A head with a forward hook, a replaced forward or a subclass's forward is called as a module."""
+    print(f"case customised_lm_head {how}", flush=True)
+    model = _tiny(dev)
+    install(model, "dense_rd", **KW)
+    head = model.lm_head
+    if how == "hook":
+        head.register_forward_hook(lambda m, args, out: out * 2)
+    elif how == "forward":
+        head.forward = lambda x: 2 * torch.nn.functional.linear(x, head.weight)
+    else:
+        class Doubled(torch.nn.Linear):
+            def forward(self, x):
+                return 2 * super().forward(x)
+
+        head.__class__ = Doubled
+    dec, _, _ = graph_prefill(model, _ids(dev), 8, headroom=64)
+    dec.run(1)
+    doubled = dec.logits.clone()
+    plain = _tiny(dev)
+    install(plain, "dense_rd", **KW)
+    dec, _, _ = graph_prefill(plain, _ids(dev), 8, headroom=64)
+    dec.run(1)
+    # logits of one bf16 product each, rounded once per product order: 2^-8 of the largest
+    assert (doubled.float() - 2 * dec.logits.float()).abs().max() <= 2 * 2 ** -7 * dec.logits.float().abs().max()
+
+
 def test_generate_eos_and_rewind(dev):
     print("case generate_eos", flush=True)
     model = _tiny(dev)

@@ -86,6 +86,12 @@ def _plain_linear(m):
     return isinstance(m, torch.nn.Linear) and m.bias is None
 
 
+def _uncustomised(m):
+    """Whether calling the Linear m runs Linear.forward and nothing else: no hooks, no forward of its own."""
+    return (not m._forward_hooks and not m._forward_pre_hooks
+            and getattr(m.forward, "__func__", None) is torch.nn.Linear.forward)
+
+
 class _LayerPlan:
     """What a decode step needs of one decoder layer, resolved once."""
 
@@ -333,9 +339,9 @@ class StaticDecoder:
 
     def _head(self, hid, res):
         """lm_head on the final norm of hid + res (res None: hid) -> [vocab]; one bb_gemv_norm launch where the modules
-        allow."""
+        allow (a head with hooks or a forward of its own is called)."""
         head, f = self.model.lm_head, self._fast_norm(self.core.norm, hid)
-        if (f and _plain_linear(head) and gemv_ok(head.weight, hid) and hid.shape[-1] <= 8192
+        if (f and _plain_linear(head) and _uncustomised(head) and gemv_ok(head.weight, hid) and hid.shape[-1] <= 8192
                 and (res is None or (res.dtype == hid.dtype and res.numel() == hid.numel()))):
             return linear_vec_norm(hid, res, *f, head.weight)[1][0, -1]
         _, x = self._add_norm(self.core.norm, hid, res)
