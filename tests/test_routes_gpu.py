@@ -157,6 +157,29 @@ def test_score_workgroups_bit_exact(T, H, Hkv, d, nr, dtype, dev):
     assert torch.equal(pooled.cpu()[:, sink:T - window], prob[:, sink:T - window])
 
 
+@pytest.mark.parametrize("T", [1016, 1025, 1031, 1032, 1033, 1039, 2057, 3087])
+@pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16), (32, torch.bfloat16)],
+                         ids=["mfma", "fp16", "chains"])
+def test_row_sums_at_score_row_ends(T, d, dtype, dev):
+    """Row sums where a score row ends inside a lane's 16 keys, over scratch memory that held large scores before: the
+    keys past T add nothing, bit for bit."""
+    print(f"case row_sum_ends T={T} d={d} {dtype}", flush=True)
+    H, Hkv, sink, window, budget = 8, 2, 8, 64, 32
+    inp = make_inputs(T, H, Hkv, d, seed=T, window=window, sink=sink, dtype=dtype)
+    q, k = inp["q"], inp["k"]
+    gq, gk = q.to(dev), k.to(dev)
+    for words in (1 << 20, 1 << 22):
+        junk = torch.full((words,), 30000.0, dtype=dtype, device=dev)
+        del junk
+    idx, pooled = hip_routes(gq, gk, num_heads=H, num_kv_heads=Hkv, sink=sink, window=window, budget=budget,
+                             n_route=64, scaling=d ** -0.5, return_pooled=True)
+    want, want_pooled = oracle.routes(q[0], k[0], sink=sink, window=window, budget=budget, scaling=d ** -0.5, n_route=64,
+                                      route_pool="mean", qpos=torch.arange(T - 64, T), return_pooled=True)
+    assert torch.equal(idx.cpu(), want)
+    prob = (want_pooled.double() * 2.0 ** -40 / 64).float()
+    assert torch.equal(pooled.cpu()[:, sink:T - window], prob[:, sink:T - window])
+
+
 @pytest.mark.parametrize("heads", [(32, 8), (32, 16), (32, 32)], ids=["gqa4", "gqa2", "mha"])
 def test_mfma_scores_d64_match_reference_order(heads, dev, monkeypatch):
     """head_dim 64 on MFMA with exact fix-up against every score in the reference order, rows and keys over many binades."""
