@@ -315,3 +315,35 @@ def test_decode_step_in_graph(dev):
         assert torch.equal(out_g, eager[i][0]), i
         _ = torch.zeros(1, device=dev).sum().item()  # unrelated eager work between replays
     assert torch.equal(kg, ke) and torch.equal(vg, ve)
+
+
+@pytest.mark.parametrize("call", ["one_token", "decode_step"])
+@pytest.mark.parametrize("n", [257, 4099, 8192])  # 2, 17 and 32 splits: the merge takes 16 (head_dim 128) or 32 a step
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float16, 128),
+                                     (torch.float16, 64)])
+def test_infinite_value_stays_in_its_column(dtype, d, n, call, dev):
+    """One token over a cache with an infinite V value in the first split: its column is infinite for the KV head's
+    query heads and every other output is bit for bit what it is without that value (no split that does not exist is
+    weighted by zero)."""
+    print(f"case infinite_value {call} {dtype} d={d} n={n}", flush=True)
+    from bigger_bird_amd import decode_bf16
+    from bigger_bird_amd.decode import decode_dense, decode_step
+
+    h, hk = 32, 8
+    g = torch.Generator(device=dev).manual_seed(n + d)
+    k, v = (torch.randn(hk, n, d, device=dev, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(h, d, device=dev, generator=g).to(dtype)
+
+    def run(v):
+        if call == "decode_step":
+            new = [x[:, -1].clone() for x in (k, v)]
+            return decode_step(q, k.clone(), v.clone(), *new, torch.tensor([n], device=dev), scale=d ** -0.5)
+        return (decode_bf16 if dtype == torch.bfloat16 else decode_dense)(q, k, v, d ** -0.5)
+
+    want = run(v)
+    v = v.clone()
+    v[3, 5, 7] = float("inf")
+    got = run(v)
+    hit = torch.zeros(h, d, dtype=torch.bool, device=dev)
+    hit[12:16, 7] = True
+    assert torch.isposinf(got[hit]).all() and torch.equal(got[~hit], want[~hit])

@@ -285,14 +285,16 @@ __global__ __launch_bounds__(kSdMergeThreads) void sparse_merge_kernel(SparseDec
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int s = s0 + u * NG;
-      const float* row = base + (int64_t)(s < p.n_splits ? s : 0) * (D + 2);
-      mv[u] = s < p.n_splits ? row[D] : -1.0e30f;
-      lv[u] = row[D + 1];
-      ov[u] = row[d];
+      const bool ok = s < p.n_splits;
+      const float* row = base + (int64_t)(ok ? s : 0) * (D + 2);
+      const float rm = row[D], rl = row[D + 1], ro = row[d];
+      mv[u] = ok ? rm : -1.0e30f;  // zeros in place of the stand-in row's values: its infinity times zero would be NaN
+      lv[u] = ok ? rl : 0.0f;
+      ov[u] = ok ? ro : 0.0f;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const float w = s0 + u * NG < p.n_splits ? fast_exp2(mv[u] - M) : 0.0f;
+      const float w = fast_exp2(mv[u] - M);
       L += w * lv[u];
       O += w * ov[u];
     }
