@@ -159,6 +159,20 @@ def test_split_chunks(t, n, front, window, noncausal, heads, d, dev):
     _check(out, ref, "split_chunks")
 
 
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("stride", [0, 8, 24])
+def test_key_rows_closer_than_head_dim(stride, d, dev):
+    """K rows that overlap (a row stride below head_dim, or 0: one row for all positions) read as any other view."""
+    print(f"case overlapping_rows stride={stride} d={d}", flush=True)
+    H, Hkv, n, front, window, rk = 8, 2, 300, 16, 64, 32
+    q, v, idx = _rand((H, n, d), 32), _rand((Hkv, n, d), 33), _routes(H, n, front, window, rk, 34)
+    base = _rand((Hkv, n * stride + d), 31).to(dev)  # a multiple of 8 elements per head
+    k = base.as_strided((Hkv, n, d), (base.shape[1], stride, 1))
+    kw = dict(front=front, window=window, num_heads=H, kv_groups=H // Hkv, scale=d ** -0.5)
+    out = bigger_bird_flash(q.to(dev), k, v.to(dev), idx.to(dev), **kw)
+    _check(out, oracle.attn_all(q, k.cpu().contiguous(), v, idx, **kw), "overlapping_rows")
+
+
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float16, 64)])
 def test_split_chunks_infinite_value(dtype, d, dev):
     """An infinite value in the first key chunk reaches its column as infinity and leaves the others alone: the merge

@@ -903,9 +903,10 @@ __global__ __launch_bounds__(256) void route_tiles_kernel(FlashParams p, uint16_
 bool flash_pipe_supported(const FlashParams& p, int D, int hpw) {
   // Buffer offsets are unsigned 32-bit: every K offset up to the end of the last tile (row N + 63, which reads as
   // zero) and every V^T offset of one KV head must stay below 4 GiB, so that no offset wraps back into the
-  // tensor. Split mode needs whole tiles.
+  // tensor. The K resource ends after N row strides, so rows that overlap (a stride below D, as of an expanded view)
+  // would lose the end of the last ones: they take the generic kernel. Split mode needs whole tiles.
   const int64_t lim = (int64_t)1 << 32;
-  const bool fits = (p.N + kTileKeys) * p.sk1 * 2 < lim && (int64_t)D * p.np * 2 < lim;
+  const bool fits = p.sk1 >= D && (p.N + kTileKeys) * p.sk1 * 2 < lim && (int64_t)D * p.np * 2 < lim;
   const bool chunks_ok = p.n_chunks == 1 || (p.key_chunk % kTileKeys == 0 && p.route_k == 0);
   // 4, 2 or 1 query heads per workgroup; the in-kernel gather of several route groups is built for 4
   const bool heads_ok = (hpw == 4 || hpw == 2 || hpw == 1) && p.G % hpw == 0 &&
