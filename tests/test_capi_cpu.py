@@ -49,6 +49,19 @@ def test_version_and_sizes():
     assert L.bb_sparse_flash_workspace(32, 131072, 131072, 128, 32, 4, 64, 16384, 512, 1, 131072, 1, 1) == 0
 
 
+@pytest.mark.parametrize("T,N,front,window", [(512, 131072, 0, 4096), (256, 131072, 64, 4096), (1024, 131072, 64, 8192),
+                                              (256, 32768, 64, 4096), (256, 1048576, 64, 16384), (65, 20011, 4096, 512)])
+def test_windowed_split_stays_in_one_round(T, N, front, window):
+    """Few rows, a window shorter than the keys, no routes: the key chunks of all row tiles (64 rows of one KV head's 4
+    query heads) fill the 256 CUs at most once, and the partials hold no more than those chunks."""
+    L = _lib.lib()
+    bytes_ = L.bb_sparse_flash_workspace(32, T, N, 128, 32, 4, front, window, 0, 1, T, 1, 0)
+    chunks = bytes_ // (32 * T * (128 + 2) * 4)
+    assert 8 * -(-T // 64) * chunks <= 256
+    # a front and a window that the call refuses: the query still answers
+    assert L.bb_sparse_flash_workspace(32, T, N, 128, 32, 4, -191, 1, 0, 1, T, 1, 0) >= 0
+
+
 def _flash_call(**over):
     L = _lib.lib()
     s3 = _lib.i64s(4096, 128, 1)

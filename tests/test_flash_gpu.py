@@ -159,6 +159,25 @@ def test_split_chunks(t, n, front, window, noncausal, heads, d, dev):
     _check(out, ref, "split_chunks")
 
 
+@pytest.mark.parametrize("H,Hkv,d,t,n,front,window", [
+    (8, 2, 128, 130, 4000, 200, 900), (8, 4, 128, 300, 5000, 64, 512), (4, 4, 128, 513, 3000, 0, 256),
+    (8, 2, 64, 65, 6000, 333, 1025), (8, 2, 64, 700, 700, 100, 300),  # the last: first rows before the window's start
+    (8, 2, 32, 130, 4000, 200, 900), (32, 8, 128, 256, 20000, 64, 4096), (8, 2, 128, 64, 2000, 1500, 300)])
+@pytest.mark.parametrize("masked", [False, True], ids=["open", "masked"])
+def test_window_chunks(H, Hkv, d, t, n, front, window, masked, dev):
+    """Few rows, a window shorter than the keys, no routes: the chunks of a row tile cover its front and window tiles
+    alone. Pipelined kernel, and the generic one (head_dim 32, or a token mask); against the float64 oracle."""
+    print(f"case window_chunks {H}/{Hkv} d={d} t={t} n={n} front={front} window={window} {masked}", flush=True)
+    q, k, v = _rand((H, t, d), 41), _rand((Hkv, n, d), 42), _rand((Hkv, n, d), 43)
+    none = torch.empty(H, 1, 0, dtype=torch.int32, device=dev)
+    kw = dict(front=front, window=window, num_heads=H, kv_groups=H // Hkv, scale=d ** -0.5)
+    tm = torch.ones(1, n, dtype=torch.bool)
+    tm[0, n - window // 2: n - window // 2 + 40] = tm[0, :3] = not masked
+    out = bigger_bird_flash(q.to(dev), k.to(dev), v.to(dev), none, token_mask=tm.to(dev) if masked else None, **kw)
+    ref = oracle.attn_all(q, k, v, torch.full((H, 1, 1), -1, dtype=torch.int32), token_mask=tm, **kw)
+    _check(out, ref, "window_chunks")
+
+
 @pytest.mark.parametrize("d", [32, 64, 128])
 @pytest.mark.parametrize("stride", [0, 8, 24])
 def test_key_rows_closer_than_head_dim(stride, d, dev):

@@ -52,8 +52,8 @@ bool flash_pipe_enabled() {
   return on;
 }
 
-FlashSchedule flash_schedule(int BH, int64_t T, int64_t N, int D, int kv_groups, int64_t window, int route_k,
-                             int64_t row_end) {
+FlashSchedule flash_schedule(int BH, int64_t T, int64_t N, int D, int kv_groups, int64_t front, int64_t window,
+                             int route_k, int64_t row_end) {
   FlashSchedule s;
   const int G = kv_groups;
   s.hpw = (G % 4 == 0) ? 4 : (G % 2 == 0) ? 2 : 1;
@@ -63,19 +63,23 @@ FlashSchedule flash_schedule(int BH, int64_t T, int64_t N, int D, int kv_groups,
   s.row_tiles = (int)cdiv(rows > 0 ? rows : 0, R);
   const int64_t n_kvbh = BH / G;
   const int64_t items = n_kvbh * s.head_splits * s.row_tiles;
-  int64_t span = (window < N ? window : N) + R;  // keys per item (window part)
   s.split = false;
   s.n_chunks = 1;
   s.key_chunk = N;
   // Few items (the exact tail, a few new rows over a long cache) leave most of the 256 CUs idle, one workgroup per CU:
-  // cut their key range into chunks, at most as many as fill the chip once (a second round of workgroups costs a
+  // cut their key tiles into chunks, at most as many as fill the chip once (a second round of workgroups costs a
   // second prologue and epilogue: the 128K tail 0.42 ms with 8 chunks, 0.46 with 16). The count is the one with the
   // least modelled time, in key tiles of one workgroup (about 1.1 us each when the chip is not full): the tiles of a
   // chunk, 4 for the merge launch, and 1 per 2.2 MB of fp32 partials written and read back. Chunks used to be at
   // least 4096 keys long: 65 rows over 20000 keys 99 -> 41 us, 256 over 8111 150 -> 46 us, 256 over 4096 80 -> 36 us,
   // 2 over 1024 25 -> 17 us; a causal prompt of 777 rows (2 chunks 40 us, none 25 us) stays whole by the partials.
   if (route_k == 0 && items > 0 && items < kCUs) {
-    const int64_t tiles = cdiv(span, 64), most = std::min<int64_t>(kCUs / items, tiles / 4);
+    // The most key tiles a row tile attends: its front tiles and the ones its rows' windows touch. With a window the
+    // chunks cut that list (chunk_tiles), not all N keys, so that no chunk lies outside the window.
+    const int64_t all = cdiv(N, 64);
+    const int64_t list =  // at least 1: the workspace query also sees arguments that the call refuses
+        window < N ? std::max<int64_t>(1, std::min(all, cdiv(front, 64) + cdiv(window + R + 62, 64))) : all;
+    const int64_t tiles = window < N ? list : cdiv(N + R, 64), most = std::min<int64_t>(kCUs / items, tiles / 4);
     const double part_tiles = (double)BH * (double)rows * (D + 2) * sizeof(float) / 2.2e6;
     double best = (double)tiles;
     int64_t nc = 1;
@@ -86,18 +90,10 @@ FlashSchedule flash_schedule(int BH, int64_t T, int64_t N, int D, int kv_groups,
         nc = c;
       }
     }
-    if (nc > 1) {
-      // chunks of the keys a workgroup attends; with a window shorter than N the chunk grid still covers all N keys
-      // (workgroups of the chunks outside the window end at once), so it has at most 64 chunks then
-      const int64_t keys = window < N ? std::max(cdiv(span, nc), cdiv(N, 64)) : cdiv(N, nc);
-      s.key_chunk = cdiv(keys, 64) * 64;
-      s.n_chunks = (int)cdiv(N, s.key_chunk);
-      s.split = s.n_chunks > 1;
-      if (!s.split) {
-        s.n_chunks = 1;
-        s.key_chunk = N;
-      }
-    }
+    const int64_t chunk = cdiv(list, nc);  // tiles per chunk
+    s.n_chunks = (int)cdiv(list, chunk);
+    s.split = s.n_chunks > 1;
+    if (s.split) s.key_chunk = chunk * 64;
   }
   return s;
 }
@@ -164,7 +160,7 @@ size_t bb_sparse_flash_workspace(int BH, int64_t T, int64_t N, int D, int num_he
   if (BH <= 0 || T <= 0 || N <= 0 || kv_groups <= 0 || BH % kv_groups) return 0;
   if (window >= N) route_k = 0;
   if (row_end <= 0 || row_end > T) row_end = T;
-  FlashSchedule s = flash_schedule(BH, T, N, D, kv_groups, window, route_k, row_end);
+  FlashSchedule s = flash_schedule(BH, T, N, D, kv_groups, front, window, route_k, row_end);
   size_t bytes = 0;
   if (!have_vt) bytes += align256((size_t)(BH / kv_groups) * D * bb_transpose_v_cols(N) * 2);
   if (routed_tiles_wanted(D, kv_groups, route_k, n_groups, has_key_mask != 0))
@@ -219,7 +215,7 @@ static int sparse_flash_impl(const void* q, const int64_t* sq, const void* k, co
   // A routed key j is attended only when j <= q - window; with window >= N no key qualifies, so the routes are
   // dropped (this is how the exact tail calls the kernel: window = N with a -1 route list).
   if (window >= N) route_k = 0;
-  FlashSchedule s = flash_schedule(BH, T, N, D, kv_groups, window, route_k, row_end);
+  FlashSchedule s = flash_schedule(BH, T, N, D, kv_groups, front, window, route_k, row_end);
   bb::FlashParams p;
   memset(&p, 0, sizeof(p));
   p.q = static_cast<const uint16_t*>(q);

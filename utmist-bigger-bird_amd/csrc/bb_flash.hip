@@ -164,7 +164,15 @@ __global__ __launch_bounds__(64 * NW, 1) void flash_kernel(FlashParams p) {
   const int64_t qw0 = p.offset + rw * p.pos_step;
   const int64_t qw1 = p.offset + (rw + RW - 1 < r1 ? rw + RW - 1 : r1) * p.pos_step;
   const uint8_t* km = HAS_MASK ? p.key_mask + (int64_t)batch * p.smb : nullptr;
-  if (SPLIT && chunk_unused(p, chunk, qlo, qhi)) return;  // the merge skips it
+  // ---- tile ranges (64-aligned): front tiles then window tiles ----
+  const TileRanges tr = tile_ranges(p, qlo, qhi);
+  int64_t c0 = 0, c1 = qhi / kTileKeys + 1;
+  if (SPLIT) {
+    int64_t ce;
+    chunk_tiles(p, chunk, tr, c0, ce);
+    if (tiles_unused(p, c0, ce, qlo, qhi)) return;  // the merge skips it
+    if (ce < c1) c1 = ce;
+  }
 
   WaveState<D, QB> st;
 #pragma unroll
@@ -184,23 +192,7 @@ __global__ __launch_bounds__(64 * NW, 1) void flash_kernel(FlashParams p) {
   const uint16_t* vbase = p.v + (int64_t)kvbh * p.sv0;
   const uint16_t* vtbase = p.vt + (int64_t)kvbh * D * p.np;
 
-  // ---- tile ranges (64-aligned): front tiles then window tiles ----
-  const int64_t front_end = p.front < qhi + 1 ? p.front : qhi + 1;
-  int64_t wlo = qlo - p.window + 1;
-  if (wlo < 0) wlo = 0;
-  int64_t kmin = 0, kmax = qhi;
-  if (SPLIT) {
-    kmin = (int64_t)chunk * p.key_chunk;
-    const int64_t ke = kmin + p.key_chunk - 1;
-    if (ke < kmax) kmax = ke;
-  }
-  int64_t f0 = 0, f1 = front_end > 0 ? (front_end + kTileKeys - 1) / kTileKeys : 0;
-  int64_t w0 = wlo / kTileKeys, w1 = qhi / kTileKeys + 1;
-  if (w0 <= f1) {
-    f1 = 0;
-    w0 = 0;
-  }
-  const int64_t c0 = kmin / kTileKeys, c1 = kmax / kTileKeys + 1;
+  int64_t f0 = 0, f1 = tr.f1, w0 = tr.w0, w1 = qhi / kTileKeys + 1;
   if (f0 < c0) f0 = c0;
   if (f1 > c1) f1 = c1;
   if (f1 < f0) f1 = f0;
@@ -371,14 +363,19 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashParams p) {
   if (item >= (int64_t)p.BH * rows) return;
   const int bh = (int)(item / rows);
   const int64_t row = item % rows;
-  const int64_t q = p.offset + row * p.pos_step;
+  const int tile_rows = 256 * p.head_splits / p.G;  // 256 rows of the workgroup's G / head_splits query heads
+  const int64_t q = p.offset + row * p.pos_step, r0 = row - (uint32_t)row % (uint32_t)tile_rows;
+  const int64_t r1 = (r0 + tile_rows < rows ? r0 + tile_rows : rows) - 1;
+  const TileRanges tr = tile_ranges(p, p.offset + r0 * p.pos_step, p.offset + r1 * p.pos_step);
   const int64_t base0 = (int64_t)bh * p.T + row, bstep = (int64_t)p.BH * p.T;
   constexpr int PER = (D + 63) / 64, U = 8;
   float M = -1.0e30f, L = 0.0f, acc[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) acc[i] = 0.0f;
   for (int c0 = 0; c0 < p.n_chunks; c0 += 64) {
-    const bool ok = c0 + lane < p.n_chunks && !chunk_unused(p, c0 + lane, q, q);
+    int64_t k0, k1;
+    chunk_tiles(p, c0 + lane, tr, k0, k1);
+    const bool ok = c0 + lane < p.n_chunks && !tiles_unused(p, k0, k1, q, q);
     const uint64_t used = __builtin_amdgcn_ballot_w64(ok);
     if (!used) continue;
     const float2 ml = ok ? *reinterpret_cast<const float2*>(p.part_ml + 2 * (base0 + (c0 + lane) * bstep))

@@ -483,7 +483,10 @@ BB_DEV PipeItem pipe_item(const FlashParams& p, int bid, int hd, int rbk) {
 // are pre-gathered); a separate instantiation, so that the common kernel's register allocation is not affected.
 // HPW: query heads per workgroup (4 when a KV head serves a multiple of 4 query heads; 2 and 1 for 2 and 1, with
 // 4 and 8 row blocks of 32 rows), so every staged K / V^T tile is read by all 8 waves in each case.
-template <bool F16, bool GATHER, int HPW, int D>
+// LIST: split mode with a window shorter than N (chunk_tiles); an instantiation of its own, because any change of the code
+// before the loop moves the loop of the others off its place in the 64-byte instruction lines (131072 tokens 25.97 ->
+// 26.20 ms, head_dim 64 with one query head per KV head 4% slower; the same loop, instruction for instruction).
+template <bool F16, bool GATHER, int HPW, int D, bool LIST = false>
 __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) {
   constexpr int PTE = Pipe<D>::TE, PBLK = Pipe<D>::BLK;
   constexpr bool kLoadInMfmaPhase = D == 64;
@@ -553,12 +556,18 @@ __global__ __launch_bounds__(64 * PNW, 1) void flash_ping_kernel(FlashParams p) 
   // split mode (exact tail: no routes): only the tiles of key chunk `chunk`, [c0, c1)
   int64_t c0 = 0, c1 = w1 > f1 ? w1 : f1;
   if (p.n_chunks > 1) {
-    // A chunk without a tile of these rows runs no step and writes an empty partial, which the merge does not read: an
-    // early return here, before or after the loop, changed the code of the whole kernel (main pass 24.19 -> 24.27 ms,
-    // tail 0.413 -> 0.425 ms at 128K).
-    c0 = (int64_t)chunk * p.key_chunk / kTileKeys;
-    const int64_t ce = ((int64_t)chunk + 1) * p.key_chunk / kTileKeys;
-    if (ce < c1) c1 = ce;
+    // A chunk past these rows' tiles (a row tile near the first key) runs no step and writes an empty partial, which the
+    // merge does not read: an early return here, before or after the loop, moved the loop as above (main pass 24.19 ->
+    // 24.27 ms, tail 0.413 -> 0.425 ms at 128K).
+    if constexpr (LIST) {
+      int64_t ce;
+      chunk_tiles(p, chunk, TileRanges{f1, w0}, c0, ce);
+      if (ce < c1) c1 = ce;
+    } else {
+      c0 = (int64_t)chunk * p.key_chunk / kTileKeys;
+      const int64_t ce = ((int64_t)chunk + 1) * p.key_chunk / kTileKeys;
+      if (ce < c1) c1 = ce;
+    }
   }
   auto clip = [&](int64_t& lo, int64_t& hi) {
     if (lo < c0) lo = c0;
@@ -928,20 +937,29 @@ hipError_t launch_route_tiles(const FlashParams& p, int D, uint16_t* rt, hipStre
 }
 
 namespace {
+template <bool F16, int D, bool LIST>
+hipError_t launch_flash_pipe_heads(const FlashParams& p, int hpw, dim3 grid, hipStream_t stream) {
+  const dim3 block(64 * PNW);
+  if (hpw == 4) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 4, D, LIST>), grid, block, 0, stream, p);
+  else if (hpw == 2) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 2, D, LIST>), grid, block, 0, stream, p);
+  else if (hpw == 1) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 1, D, LIST>), grid, block, 0, stream, p);
+  else return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
 template <bool F16, int D>
 hipError_t launch_flash_pipe_t(const FlashParams& p, int hpw, hipStream_t stream) {
   const int64_t items = (int64_t)p.n_kvbh * p.head_splits * p.row_tiles * p.n_chunks;
   if (items <= 0) return hipSuccess;
   if (items > 0x7fffffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)items), block(64 * PNW);
-  const bool gather = p.route_k > 0 && !p.rtiles;
-  if (gather && hpw != 4) return hipErrorInvalidValue;
-  if (gather) hipLaunchKernelGGL((flash_ping_kernel<F16, true, 4, D>), grid, block, 0, stream, p);
-  else if (hpw == 4) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 4, D>), grid, block, 0, stream, p);
-  else if (hpw == 2) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 2, D>), grid, block, 0, stream, p);
-  else if (hpw == 1) hipLaunchKernelGGL((flash_ping_kernel<F16, false, 1, D>), grid, block, 0, stream, p);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+  const dim3 grid((unsigned)items);
+  if (p.route_k > 0 && !p.rtiles) {
+    if (hpw != 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((flash_ping_kernel<F16, true, 4, D>), grid, dim3(64 * PNW), 0, stream, p);
+    return hipGetLastError();
+  }
+  return p.n_chunks > 1 && p.window < p.N ? launch_flash_pipe_heads<F16, D, true>(p, hpw, grid, stream)
+                                          : launch_flash_pipe_heads<F16, D, false>(p, hpw, grid, stream);
 }
 }  // namespace
 

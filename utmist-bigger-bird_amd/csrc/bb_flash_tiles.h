@@ -69,11 +69,31 @@ struct WaveState {
 
 BB_DEV int clamp64(int64_t x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : (int)x); }
 
-// Whether key chunk `chunk` (split mode) holds no key for query positions qlo..qhi: it starts past the last of them,
-// or lies between the front and the first one's window.
-BB_DEV bool chunk_unused(const FlashParams& p, int chunk, int64_t qlo, int64_t qhi) {
-  const int64_t c0 = (int64_t)chunk * p.key_chunk;
-  return c0 > qhi || (c0 >= p.front && c0 + p.key_chunk <= qlo - p.window + 1);
+// Key tiles of query positions qlo..qhi: the front's [0, f1) and the window's, from w0 on; one range from 0 (both 0)
+// where they touch.
+struct TileRanges {
+  int64_t f1, w0;
+};
+BB_DEV TileRanges tile_ranges(const FlashParams& p, int64_t qlo, int64_t qhi) {
+  const int64_t front_end = p.front < qhi + 1 ? p.front : qhi + 1, wlo = qlo - p.window + 1;
+  const int64_t f1 = front_end > 0 ? (front_end + kTileKeys - 1) / kTileKeys : 0, w0 = wlo > 0 ? wlo / kTileKeys : 0;
+  return w0 <= f1 ? TileRanges{0, 0} : TileRanges{f1, w0};
+}
+// Split mode: a chunk is key_chunk / 64 consecutive entries of its row tile's list, the front tiles and then the window
+// tiles, as the key tiles [c0, c1). Chunks of all N keys would mostly lie outside a short window, and each would still
+// cost a workgroup and its partials: 512 rows over 131072 keys, window 4096, 32 heads over 8: 214 us and 545 MB of
+// workspace with 64 chunks of all keys, 99 us and 34 MB with 4, 52 us and 34 MB with 4 of the list.
+BB_DEV void chunk_tiles(const FlashParams& p, int chunk, const TileRanges& tr, int64_t& c0, int64_t& c1) {
+  const int64_t n = p.key_chunk / kTileKeys, gap = tr.w0 - tr.f1;
+  c0 = chunk * n;
+  c1 = c0 + n;
+  if (c0 >= tr.f1) c0 += gap;
+  if (c1 > tr.f1) c1 += gap;
+}
+// Whether key tiles [c0, c1) hold no key for query positions qlo..qhi: they start past the last of them, or lie between
+// the front and the first one's window.
+BB_DEV bool tiles_unused(const FlashParams& p, int64_t c0, int64_t c1, int64_t qlo, int64_t qhi) {
+  return c0 * kTileKeys > qhi || (c0 * kTileKeys >= p.front && c1 * kTileKeys <= qlo - p.window + 1);
 }
 
 // Window/front mask of one tile for one query row, reduced to int32 thresholds on the tile-relative key kk:
