@@ -137,6 +137,27 @@ def test_customised_lm_head_is_called(how, dev):
     assert (doubled.float() - 2 * dec.logits.float()).abs().max() <= 2 * 2 ** -7 * dec.logits.float().abs().max()
 
 
+@pytest.mark.parametrize("kind", ["forward", "pre"])
+def test_global_hooks_see_lm_head(kind, dev):
+    """A hook registered for every module runs for the head too."""
+    from torch.nn.modules import module
+
+    print(f"case global_hooks {kind}", flush=True)
+    model = _tiny(dev)
+    install(model, "dense_rd", **KW)
+    dec, _, _ = graph_prefill(model, _ids(dev), 8, headroom=64)
+    seen = []
+    if kind == "forward":
+        handle = module.register_module_forward_hook(lambda m, args, out: seen.append(m))
+    else:
+        handle = module.register_module_forward_pre_hook(lambda m, args: seen.append(m))
+    try:
+        dec.run(1, graph=False)
+    finally:
+        handle.remove()
+    assert model.lm_head in seen
+
+
 def test_generate_eos_and_rewind(dev):
     print("case generate_eos", flush=True)
     model = _tiny(dev)

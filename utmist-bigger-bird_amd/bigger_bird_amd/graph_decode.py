@@ -87,8 +87,11 @@ def _plain_linear(m):
 
 
 def _uncustomised(m):
-    """Whether calling the Linear m runs Linear.forward and nothing else: no hooks, no forward of its own."""
+    """Whether calling the Linear m runs Linear.forward and nothing else: no hooks of its own or for every module, no
+    forward of its own."""
+    every = torch.nn.modules.module
     return (not m._forward_hooks and not m._forward_pre_hooks
+            and not every._global_forward_hooks and not every._global_forward_pre_hooks
             and getattr(m.forward, "__func__", None) is torch.nn.Linear.forward)
 
 
