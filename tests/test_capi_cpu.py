@@ -185,6 +185,16 @@ def test_int8_layer_host_state_without_gpu():
     assert all(isinstance(x, Int8KVLayer) and not x.fused and x.scale_dtype == torch.float32 for x in cache.layers)
 
 
+@pytest.mark.parametrize("q,k,v", [((32, 128), (8, 300, 128), (8, 299, 128)), ((32, 128), (8, 300, 128), (4, 300, 128)),
+                                   ((32, 128), (8, 300, 64), (8, 300, 64)), ((30, 128), (8, 300, 128), (8, 300, 128))])
+def test_decode_bf16_refuses_mismatched_shapes(q, k, v):
+    """Refused before any launch, whatever the device: the kernel takes lengths and heads from K alone."""
+    from bigger_bird_amd import decode_bf16
+
+    with pytest.raises(ValueError, match="must match"):
+        decode_bf16(*(torch.zeros(s, dtype=torch.bfloat16) for s in (q, k, v)), 0.1)
+
+
 def test_decode_append_and_kv_append_argument_errors():
     """Argument checks of the decode-step entry points run before any launch (no GPU needed)."""
     L = _lib.lib()

@@ -166,6 +166,9 @@ def decode_int8_append(q, k8, ks, v8, vs, knew, vnew, n, scale, min_scale=MIN_SC
 
 def decode_bf16(q, k, v, scale):
     """q [H, d] bf16 over k/v [Hkv, n, d] (strided views of a bf16 cache)."""
+    if (q.ndim != 2 or k.ndim != 3 or k.shape != v.shape or q.shape[-1] != k.shape[-1] or not k.shape[0]
+            or q.shape[0] % k.shape[0]):
+        raise ValueError("q [H,D] and k/v [Hkv,N,D] must match")  # the kernel takes lengths and heads from k alone
     _lib.require_gpu(k, v, what="decode_bf16")
     if k.dtype != torch.bfloat16 or v.dtype != torch.bfloat16:
         raise ValueError("decode_bf16: bf16 cache required")
