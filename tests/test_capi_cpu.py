@@ -185,6 +185,18 @@ def test_int8_layer_host_state_without_gpu():
     assert all(isinstance(x, Int8KVLayer) and not x.fused and x.scale_dtype == torch.float32 for x in cache.layers)
 
 
+def test_int8_layer_first_fill_that_fails_leaves_it_empty():
+    """A first update whose rows cannot be quantised raises and leaves the layer without rows, so that the next one is
+    the first again."""
+    from bigger_bird_amd.kv_int8 import Int8KVLayer
+
+    layer = Int8KVLayer()
+    x = torch.zeros(1, 2, 5, 128, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match="ROCm device"):
+        layer.update(x, x)
+    assert layer.store_k is None and layer.store_v is None and layer.get_seq_length() == 0
+
+
 @pytest.mark.parametrize("q,k,v", [((32, 128), (8, 300, 128), (8, 299, 128)), ((32, 128), (8, 300, 128), (4, 300, 128)),
                                    ((32, 128), (8, 300, 64), (8, 300, 64)), ((30, 128), (8, 300, 128), (8, 300, 128))])
 def test_decode_bf16_refuses_mismatched_shapes(q, k, v):

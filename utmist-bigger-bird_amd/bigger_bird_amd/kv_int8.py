@@ -316,9 +316,9 @@ class Int8KVLayer(DynamicLayer):
         t = key_states.shape[-2]
         if self.store_k is None:
             kr, vr = self._token_major(key_states), self._token_major(value_states)
-            self.store_k, self.store_v = (_Int8Rows(x.shape[1], x.shape[2], t, self.scale_dtype, x.device) for x in (kr, vr))
-            quantize_pair(kr, vr, self.store_k.rows(0, t), self.store_v.rows(0, t), scale_dtype=self.scale_dtype)
-            self.n = t
+            sk, sv = (_Int8Rows(x.shape[1], x.shape[2], t, self.scale_dtype, x.device) for x in (kr, vr))
+            quantize_pair(kr, vr, sk.rows(0, t), sv.rows(0, t), scale_dtype=self.scale_dtype)
+            self.store_k, self.store_v, self.n = sk, sv, t  # only now: rows that are refused leave the layer empty
             return key_states, value_states
         start, end = self.n, self.n + t
         self.store_k.ensure(start, end)
