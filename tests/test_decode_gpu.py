@@ -347,3 +347,18 @@ def test_infinite_value_stays_in_its_column(dtype, d, n, call, dev):
     hit = torch.zeros(h, d, dtype=torch.bool, device=dev)
     hit[12:16, 7] = True
     assert torch.isposinf(got[hit]).all() and torch.equal(got[~hit], want[~hit])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("off", [1, 4, 7])
+def test_one_token_query_at_any_element(off, dtype, dev):
+    """A query whose storage starts at any element (two-byte alignment) gives what an aligned copy of it gives."""
+    print(f"case query_offset {off} {dtype}", flush=True)
+    from bigger_bird_amd import decode_bf16
+    from bigger_bird_amd.decode import decode_dense
+
+    g = torch.Generator(device=dev).manual_seed(off)
+    k, v = (torch.randn(8, 700, 128, device=dev, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(off + 32 * 128, device=dev, generator=g).to(dtype)[off:].view(32, 128)
+    f = decode_bf16 if dtype == torch.bfloat16 else decode_dense
+    assert q.data_ptr() % 16 and torch.equal(f(q, k, v, 0.09), f(q.clone(), k, v, 0.09))

@@ -69,12 +69,14 @@ BB_DEV float round_elem(float x) {
   return elem_to_f32<F16>((uint16_t)h);
 }
 
-// q row of one lane's pieces as packed pairs (DPL 16-bit values, DPL / 2 words).
+// q row of one lane's pieces as packed pairs (DPL 16-bit values, DPL / 2 words). q may start at any element: the type
+// says so, and the target takes such a load in one instruction.
+typedef u32x4_t u32x4_at2_t __attribute__((aligned(2)));
 template <int DPL>
 BB_DEV void load_q_pairs(const uint16_t* qrow, int sub, uint32_t (&qw)[DPL / 2]) {
 #pragma unroll
   for (int e0 = 0; e0 < DPL / 8; ++e0) {
-    const u32x4_t w = ld16(qrow + piece_off(sub, e0));
+    const u32x4_t w = *reinterpret_cast<const u32x4_at2_t*>(qrow + piece_off(sub, e0));
 #pragma unroll
     for (int i = 0; i < 4; ++i) qw[4 * e0 + i] = w[i];
   }
