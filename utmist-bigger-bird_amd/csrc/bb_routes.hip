@@ -306,6 +306,11 @@ template <int D>
 constexpr int kMsRowPitch = D + 8;         // bf16 elements per staged Q row (16 bytes past it: conflict-free row reads)
 constexpr int kMsTilePitch = 40;           // bf16 per score-tile row (80 bytes: conflict-free 8-byte row writes)
 
+// LDS bytes of a scores_mfma_kernel workgroup of nw waves (RouteGeom::iters counts the ones that fit a CU by it).
+constexpr int ms_lds_bytes(int D, int nw) {
+  return 32 * nw * (D + 8) * 2 + kScoreKeys * D * 6 + nw * 32 * (kMsTilePitch + kScoreKeys) * 2 + 4 + 32 * nw * 4;
+}
+
 // Weight c_d of the certification bound for element d of a D-element dot product (see above).
 template <int D>
 BB_DEV int bound_weight(int d) {
@@ -341,6 +346,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   __shared__ uint16_t flist[NW * 32 * kScoreKeys];                          // fix-ups: wave << 10 | lane << 4 | r
   __shared__ uint32_t fcount;                                               // entries of flist
   __shared__ uint32_t rmax_fix[ROWS];                                       // ordered-float max of fixed-up x
+  static_assert(sizeof(qs) + sizeof(kt) + sizeof(kf) + sizeof(st) + sizeof(flist) + sizeof(fcount) + sizeof(rmax_fix) ==
+                ms_lds_bytes(D, NW), "ms_lds_bytes");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 31, h = lane >> 5;
   const int kchunk = blockIdx.x, rblk = blockIdx.y, bkv = blockIdx.z;
@@ -1225,19 +1232,23 @@ hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, con
   return hipGetLastError();
 }
 
-RouteGeom geom(int64_t n, int H, int Hkv, int B, int r, bool f16) {
+RouteGeom geom(int64_t n, int H, int Hkv, int B, int r, int D, bool f16) {
   RouteGeom g;
   g.G = H / Hkv;
   g.rows = g.G * r;
   g.row_blocks = (g.rows + kMaxRows - 1) / kMaxRows;
-  // Key blocks per scores workgroup: as many as make one round of resident workgroups (one, two or four per CU by LDS:
-  // 8, 4 and 2 waves; two, two and three of the VALU workgroups that fp16 scores run on), since every workgroup stages
-  // its Q rows and bound weights once, but not fewer than 4 and at most 128, in multiples of 4 (a step of the VALU
-  // scorer is up to 128 keys). At 128K tokens that is 128 blocks (0.793 ms against 0.885 with 16); with 16 at the least
-  // short prompts left half of the CUs idle: whole bb_routes calls of 32 heads over 8, 2048 tokens 120 -> 76 us, 8192
-  // 132 -> 105, 8111 in fp16 293 -> 171.
+  // Key blocks per scores workgroup: as many as make one round of resident workgroups, since every workgroup stages its
+  // Q rows and bound weights once, but not fewer than 4 and at most 128, in multiples of 4 (a step of the VALU scorer is
+  // up to 128 keys). An MFMA workgroup of nw waves is resident 8 / nw times (its registers allow two waves per SIMD) or
+  // as its LDS allows: 1, 2 and 4 per CU, but 3 of 2 waves at head_dim 128 (51 KB each; with 4 the second round was a
+  // third full: 32 KV heads of one query head, 8192 tokens 107 -> 94 us, 65536 tokens 616 -> 517). The VALU workgroups
+  // of fp16 scores: 4 of 64 rows, 2 of more. Three of them fit at head_dim 128, but 3 measured no better: 32 KV heads,
+  // 8192 tokens 145 us with 4 and 157 with 3; 8 KV heads 135 with 2, 3 and 4. At 128K tokens a bf16 workgroup takes 128
+  // blocks (0.793 ms against 0.885 with 16); with 16 at the least short prompts left half of the CUs idle: whole
+  // bb_routes calls of 32 heads over 8, 2048 tokens 120 -> 76 us, 8192 132 -> 105, 8111 in fp16 293 -> 171.
   const int64_t nbkv = (int64_t)(B > 0 ? B : 1) * Hkv;
-  const int per_cu = g.rows > 128 ? (f16 ? 2 : 1) : (g.rows > 64 ? 2 : 4);
+  const int nw = g.rows <= 64 ? 2 : (g.rows <= 128 ? 4 : 8), by_lds = 160 * 1024 / ms_lds_bytes(D, nw);
+  const int per_cu = f16 ? (g.rows > 64 ? 2 : 4) : (by_lds < 8 / nw ? by_lds : 8 / nw);
   const int64_t blocks32 = (n + kScoreKeys - 1) / kScoreKeys, lanes = nbkv * g.row_blocks;
   const int64_t chunks = kCus * per_cu / lanes > 1 ? kCus * per_cu / lanes : 1;
   const int64_t it = ((blocks32 + chunks - 1) / chunks + 3) & ~(int64_t)3;
@@ -1324,7 +1335,7 @@ hipError_t launch_topk_rows(const uint64_t* keys, int rows, int64_t stride, int6
 }
 
 size_t routes_workspace_bytes(int64_t n, int H, int Hkv, int B, int r) {
-  RouteGeom g = geom(n, H, Hkv, B, r, true);  // fp16 scores have at least as many key chunks as bf16 ones
+  RouteGeom g = geom(n, H, Hkv, B, r, 128, true);  // fp16 scores have at least as many key chunks as bf16 ones
   const size_t nbkv = (size_t)B * Hkv;
   size_t s = 0;
   s += align256(nbkv * g.rows * (size_t)g.ns * 2);        // scores
@@ -1338,7 +1349,7 @@ size_t routes_workspace_bytes(int64_t n, int H, int Hkv, int B, int r) {
 
 hipError_t launch_routes(RoutesParams& p, void* ws, size_t ws_bytes, hipStream_t stream) {
   if (ws_bytes < routes_workspace_bytes(p.n, p.H, p.Hkv, p.B, p.r)) return hipErrorInvalidValue;
-  RouteGeom g = geom(p.n, p.H, p.Hkv, p.B, p.r, p.f16 != 0);
+  RouteGeom g = geom(p.n, p.H, p.Hkv, p.B, p.r, p.D, p.f16 != 0);
   const size_t nbkv = (size_t)p.B * p.Hkv;
   p.pstride = p.n;
   p.n_dev = nullptr;
