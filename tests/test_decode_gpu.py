@@ -133,6 +133,24 @@ def test_route_matches_oracle(cap, n, front, window, routed, dtype, device_n, d,
         assert a == sorted(order.tolist()), kv
 
 
+@pytest.mark.parametrize("cap", [16384 + 32, 16384 + 33])
+def test_route_at_the_one_launch_limit(cap, dev):
+    """The longest range whose top-k is one launch (no histogram from the pool pass) and one key more, on a workspace full
+    of other bytes: the top-k of the kernel's own probabilities, ties to the lower index."""
+    print(f"case route_limit cap={cap}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(cap)
+    k = torch.randn(8, cap, 128, device=dev, generator=g).to(torch.bfloat16)
+    q = torch.randn(32, 128, device=dev, generator=g).to(torch.bfloat16)
+    kw = dict(front=32, window=64, scale=128 ** -0.5)
+    for _ in range(3):
+        junk = torch.full((1 << 24,), 0x5a, dtype=torch.uint8, device=dev)  # the allocator hands these bytes on
+        del junk
+        idx = bigger_bird_route(q, k, 200, **kw).cpu()
+    p = pooled_probs(q, k, **kw).cpu()[:, 32:cap - 64]
+    want = torch.argsort(-p, dim=-1, stable=True)[:, :200].sort(-1).values + 32
+    assert torch.equal(idx.long(), want)
+
+
 def test_route_fewer_eligible_than_budget(dev):
     """Fewer eligible keys than k_route: all of them, ascending, then -1."""
     h, hk, d, n = 8, 2, 64, 300

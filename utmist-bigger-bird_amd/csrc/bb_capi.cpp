@@ -652,7 +652,8 @@ static int route_impl(const void* q, int64_t sq, const void* k, const int64_t* s
   if (k_route > 0) {
     p.keys = reinterpret_cast<uint64_t*>(w);
     w += align256((size_t)Hkv * cap * 8);
-    bb::topk_hist_meta(w, cap, Hkv, &p.top_hist, &p.top_meta);  // filled by the pool pass
+    // filled by the pool pass, where the top-k reads it (16384 keys, 512 routed: the step 42.9 -> 42.0 us)
+    if (!bb::topk_one_launch(cap - front)) bb::topk_hist_meta(w, cap, Hkv, &p.top_hist, &p.top_meta);
   }
   if (app) p.app = *app;
   int rc = hip_status(bb::launch_decode_route_probs(p, st), "bb_decode_route");

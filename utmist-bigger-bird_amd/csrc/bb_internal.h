@@ -163,6 +163,9 @@ hipError_t launch_decode_route_probs(const DecodeRouteParams& p, hipStream_t str
 // (topk_hist_meta) were already filled and cleared by the producer of the keys.
 constexpr int kTopFloatKeys = 1, kTopHistReady = 2;
 size_t topk_workspace_bytes(int64_t stride, int rows);
+// Whether launch_topk_rows chooses among this many keys (stride - front) in one launch, which reads no histogram from the
+// workspace.
+bool topk_one_launch(int64_t range);
 void topk_hist_meta(void* ws, int64_t stride, int rows, uint32_t** hist, uint32_t** meta);
 hipError_t launch_topk_rows(const uint64_t* keys, int rows, int64_t stride, int64_t n, const int64_t* n_dev,
                             int front, int window, int budget, int32_t* out, void* ws, size_t ws_bytes, int flags,

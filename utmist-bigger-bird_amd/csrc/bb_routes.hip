@@ -63,7 +63,8 @@ struct RouteGeom {
   int iters;  // key blocks of kScoreKeys per scores workgroup: n_kb1 = ceil(n / (kScoreKeys iters))
   int sum_rows, sum_splits;  // rowsum_kernel: rows per workgroup (a multiple of 4) and row slices
   int64_t ns;  // score row stride: n rounded up to 8 (16-byte aligned rows)
-  uint32_t* top_hist;  // [B * H][kTopBins] and [B * H][kTopMetaWords]: cleared by the scorer for the top-k kernels
+  uint32_t* top_hist;  // [B * H][kTopBins] and [B * H][kTopMetaWords]: cleared by the scorer for the top-k kernels (of
+                       // ranges above kTopSmall; 8 KB a head, and a branch around it would move the scorer's loop)
   uint32_t* top_meta;
 };
 
@@ -1221,7 +1222,7 @@ hipError_t launch_routes_d(RoutesParams& p, const RouteGeom& g, float* pmax, con
     const int64_t cnt = hi > lo ? hi - lo : 0;
     const unsigned chunks = (unsigned)((cnt + kTopChunk - 1) / kTopChunk);
     const int heads = p.B * p.H;
-    if (cnt <= kTopSmall) {
+    if (topk_one_launch(cnt)) {
       hipLaunchKernelGGL(topk_small_kernel, dim3(heads), dim3(kTopThreads), 0, stream, p);
       return hipGetLastError();
     }
@@ -1292,6 +1293,8 @@ __global__ __launch_bounds__(256) void topk_clear_kernel(TopWs w) {
 
 }  // namespace
 
+bool topk_one_launch(int64_t range) { return range <= kTopSmall; }
+
 size_t topk_workspace_bytes(int64_t stride, int rows) { return top_ws_bytes(stride, (size_t)rows); }
 
 void topk_hist_meta(void* ws, int64_t stride, int rows, uint32_t** hist, uint32_t** meta) {
@@ -1321,7 +1324,7 @@ hipError_t launch_topk_rows(const uint64_t* keys, int rows, int64_t stride, int6
   const int64_t lo = front > 0 ? front : 0;
   const int64_t cnt = stride > lo ? stride - lo : 0;
   const unsigned chunks = (unsigned)((cnt + kTopChunk - 1) / kTopChunk);
-  if (cnt <= kTopSmall) {  // whatever the device length: the range is at most cnt
+  if (topk_one_launch(cnt)) {  // whatever the device length: the range is at most cnt
     hipLaunchKernelGGL(topk_small_kernel, dim3(rows), dim3(kTopThreads), 0, stream, p);
     return hipGetLastError();
   }
