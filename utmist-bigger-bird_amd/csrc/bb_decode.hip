@@ -875,23 +875,23 @@ __global__ __launch_bounds__(64 * kGvWaves) void gemv_kernel(const uint16_t* __r
 }
 
 template <int D, int GR, bool F16>
-hipError_t launch_sparse_decode_t(const SparseDecodeParams& p, hipStream_t stream) {
+hipError_t launch_sparse_decode_t(const SparseDecodeParams& p, bool merge, hipStream_t stream) {
   if (p.xs)
     hipLaunchKernelGGL((sparse_decode_kernel<D, GR, F16, true>), dim3(p.n_splits, p.rows), dim3(kSdThreads), 0, stream, p);
   else
     hipLaunchKernelGGL((sparse_decode_kernel<D, GR, F16, false>), dim3(p.n_splits, p.rows), dim3(kSdThreads), 0, stream,
                        p);
-  hipLaunchKernelGGL((sparse_merge_kernel<D, F16>), dim3(p.H), dim3(kSdMergeThreads), 0, stream, p);
+  if (merge) hipLaunchKernelGGL((sparse_merge_kernel<D, F16>), dim3(p.H), dim3(kSdMergeThreads), 0, stream, p);
   return hipGetLastError();
 }
 
 template <int D, bool F16>
-hipError_t launch_sparse_decode_d(const SparseDecodeParams& p, hipStream_t stream) {
+hipError_t launch_sparse_decode_d(const SparseDecodeParams& p, bool merge, hipStream_t stream) {
   switch (p.rows == p.H ? 1 : p.G) {
-    case 1: return launch_sparse_decode_t<D, 1, F16>(p, stream);
-    case 2: return launch_sparse_decode_t<D, 2, F16>(p, stream);
-    case 4: return launch_sparse_decode_t<D, 4, F16>(p, stream);
-    case 8: return launch_sparse_decode_t<D, 8, F16>(p, stream);
+    case 1: return launch_sparse_decode_t<D, 1, F16>(p, merge, stream);
+    case 2: return launch_sparse_decode_t<D, 2, F16>(p, merge, stream);
+    case 4: return launch_sparse_decode_t<D, 4, F16>(p, merge, stream);
+    case 8: return launch_sparse_decode_t<D, 8, F16>(p, merge, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -917,11 +917,12 @@ hipError_t launch_route_d(const DecodeRouteParams& p, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_sparse_decode(const SparseDecodeParams& p, hipStream_t stream) {
+hipError_t launch_sparse_decode(const SparseDecodeParams& p, hipStream_t stream, bool merge) {
   if (p.n_splits <= 0 || p.rows <= 0) return hipErrorInvalidValue;
-  if (p.D == 64) return p.f16 ? launch_sparse_decode_d<64, true>(p, stream) : launch_sparse_decode_d<64, false>(p, stream);
+  if (p.D == 64)
+    return p.f16 ? launch_sparse_decode_d<64, true>(p, merge, stream) : launch_sparse_decode_d<64, false>(p, merge, stream);
   if (p.D == 128)
-    return p.f16 ? launch_sparse_decode_d<128, true>(p, stream) : launch_sparse_decode_d<128, false>(p, stream);
+    return p.f16 ? launch_sparse_decode_d<128, true>(p, merge, stream) : launch_sparse_decode_d<128, false>(p, merge, stream);
   return hipErrorInvalidValue;
 }
 

@@ -741,9 +741,11 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
   if (p.knew != nullptr && !decode_fuses_append(p)) return hipErrorInvalidValue;
   if (!p.k8) {
     // A bf16 cache runs on the split-K sparse decode kernel with every key in its window: rows streamed with
-    // line-covering non-temporal loads, two keys per slot in flight. Against the one-key-per-step kernel this used to
-    // be (whole calls, us): 131072 keys of 8 KV heads x 4 query heads 97 -> 91, 16 x 2 180 -> 161, 32 x 1 355 -> 309,
-    // 4 x 8 122 -> 99; 16384 keys of 32 x 1 51 -> 48; the same below 4096 keys, where the launches are the time.
+    // line-covering non-temporal loads, two keys per slot in flight. Against the one-key-per-step kernel this used to be
+    // (us a call, caches that rotate past the 256 MB cache): 131072 keys of 8 KV heads x 4 query heads 105 -> 95, 16 x 2
+    // 191 -> 170, 32 x 1 380 -> 325, 4 x 8 124 -> 94; 16384 keys 21.7 -> 21.1, 31.4 -> 29.3, 53.6 -> 49.2, 27.1 -> 21.8.
+    // The partials (same layout) merge as those of the INT8 kernels: sparse_merge_kernel, one workgroup per query head,
+    // takes longer over 64 splits (16384 keys of 8 KV heads 23.2 us with it).
     SparseDecodeParams s = {};
     s.q = p.q; s.k = p.kb; s.v = p.vb; s.out = p.out; s.part = p.part;
     s.sq = p.sq; s.sk0 = p.skb0; s.sk1 = p.skb1; s.sv0 = p.svb0; s.sv1 = p.svb1; s.so = p.so;
@@ -752,7 +754,12 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
     s.H = p.H; s.Hkv = p.Hkv; s.G = p.H / p.Hkv; s.D = p.D; s.rows = p.Hkv;
     s.window = p.n;
     s.c = p.c;
-    return launch_sparse_decode(s, stream);
+    const hipError_t e = launch_sparse_decode(s, stream, false);
+    if (e != hipSuccess) return e;
+    const dim3 grid(p.H, p.D / kMergeCols);
+    if (p.D == 64) hipLaunchKernelGGL(decode_merge_kernel<64>, grid, dim3(kMergeThreads), 0, stream, p);
+    else hipLaunchKernelGGL(decode_merge_kernel<128>, grid, dim3(kMergeThreads), 0, stream, p);
+    return hipGetLastError();
   }
   switch (p.D) {
     case 64: return launch_decode_d<64>(p, stream);

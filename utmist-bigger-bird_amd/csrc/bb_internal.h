@@ -136,7 +136,7 @@ struct SparseDecodeParams {
   const float* xs;       // scores of this query from decode routing ([H][xs_stride], scale * log2(e) applied), or null
   int64_t xs_stride;
 };
-hipError_t launch_sparse_decode(const SparseDecodeParams& p, hipStream_t stream);
+hipError_t launch_sparse_decode(const SparseDecodeParams& p, hipStream_t stream, bool merge = true);
 
 // Decode routing: pooled probabilities over the cached keys for one query token.
 struct DecodeRouteParams {
