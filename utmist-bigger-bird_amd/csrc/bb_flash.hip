@@ -363,10 +363,13 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashParams p) {
   if (item >= (int64_t)p.BH * rows) return;
   const int bh = (int)(item / rows);
   const int64_t row = item % rows;
-  const int tile_rows = 256 * p.head_splits / p.G;  // 256 rows of the workgroup's G / head_splits query heads
-  const int64_t q = p.offset + row * p.pos_step, r0 = row - (uint32_t)row % (uint32_t)tile_rows;
-  const int64_t r1 = (r0 + tile_rows < rows ? r0 + tile_rows : rows) - 1;
-  const TileRanges tr = tile_ranges(p, p.offset + r0 * p.pos_step, p.offset + r1 * p.pos_step);
+  const int64_t q = p.offset + row * p.pos_step;
+  TileRanges tr = {0, 0};
+  if (p.window < p.N) {  // the list of the row's tile; without a window it starts at key 0 whatever the row
+    const int tile_rows = 256 * p.head_splits / p.G;  // 256 rows of the workgroup's G / head_splits query heads
+    const int64_t r0 = row - (uint32_t)row % (uint32_t)tile_rows, r1 = (r0 + tile_rows < rows ? r0 + tile_rows : rows) - 1;
+    tr = tile_ranges(p, p.offset + r0 * p.pos_step, p.offset + r1 * p.pos_step);
+  }
   const int64_t base0 = (int64_t)bh * p.T + row, bstep = (int64_t)p.BH * p.T;
   constexpr int PER = (D + 63) / 64, U = 8;
   float M = -1.0e30f, L = 0.0f, acc[PER];
