@@ -133,7 +133,7 @@ def test_d64_pipelined(H, Hkv, T, N, front, window, rk, groups, dtype, dev):
 @pytest.mark.parametrize("t,n,front,window,noncausal", [
     (2, 257, 0, 257, True), (65, 1023, 0, 1023, True), (1, 4099, 0, 4099, True),  # a handful of tiles; one row
     (300, 700, 0, 700, False), (130, 2049, 0, 2049, False),  # causal rows that end inside and before later chunks
-    (64, 9000, 70, 3000, False),                             # chunks between the front and the window hold nothing
+    (64, 9000, 70, 3000, False),                             # a front and a window far past it
     (33, 5000, 0, 1000, False)])
 @pytest.mark.parametrize("heads,d", [((32, 8), 128), ((8, 4), 128), ((4, 4), 128), ((8, 2), 64)],
                          ids=["gqa4", "gqa2", "mha", "d64"])

@@ -65,7 +65,6 @@ def _check(got, ref, what):
     assert err.max().item() < 2e-2 and err.mean().item() < 2e-3, what
 
 
-# 32769 and 131329 keys: 128 splits of 257 / 1027 keys (not a multiple of the 32-key chunk), the last one short
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("size,min_scale", [(1.0, 1e-4), (1e-3, 1e-4), (1e-6, 1e-20), (1e4, 1e-4)])
 def test_quantize_near_halves(size, min_scale, dtype, dev):
@@ -89,6 +88,7 @@ def test_quantize_near_halves(size, min_scale, dtype, dev):
     assert np.array_equal(s.cpu().numpy(), want_s) and np.array_equal(q.cpu().numpy(), want_q)
 
 
+# 32769 and 131329 keys: 64 splits of 513 / 2053 keys (not a multiple of the 32-key chunk), the last one short
 @pytest.mark.parametrize("n,H,Hkv,d,f16", [(1, 32, 8, 128, True), (300, 32, 8, 128, True), (4099, 32, 8, 128, False),
                                            (20000, 16, 2, 64, True), (32769, 32, 8, 128, True),
                                            (131072, 32, 8, 128, False), (131329, 32, 8, 128, False)])
