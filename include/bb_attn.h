@@ -34,7 +34,8 @@ extern "C" {
  *   202  bb_int8_quantize / bb_int8_quantize_pair take an element kind (0 bf16, 1 fp32, 2 fp16) where they took
  *        x_is_f32, and bb_int8_dequantize an output kind where it took out_is_f32 (the old values keep their
  *        meaning)
- *   203  bb_add_rms_norm, bb_silu_mul, bb_gemv and bb_gemv_norm added */
+ *   203  bb_add_rms_norm, bb_silu_mul, bb_gemv and bb_gemv_norm added; later, with no parameter list changed and so
+ *        under the same number, bb_gemv_norm_rope and bb_argmax_step (a library built before them lacks the symbols) */
 #define BB_ABI_VERSION 203
 int bb_version(void);
 
