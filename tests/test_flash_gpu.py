@@ -192,6 +192,35 @@ def test_key_rows_closer_than_head_dim(stride, d, dev):
     _check(out, oracle.attn_all(q, k.cpu().contiguous(), v, idx, **kw), "overlapping_rows")
 
 
+@pytest.mark.parametrize("heads", [(8, 2), (8, 4), (4, 4)], ids=["gqa4", "gqa2", "mha"])
+@pytest.mark.parametrize("routed", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_d64_infinite_value_reaches_no_far_row(heads, routed, dtype, dev):
+    """head_dim 64: an infinite V value reaches no row before its key but those of the 32-row waves that meet the key's
+    64-key tile, no row past its window where no route holds it, and it does reach rows that attend it."""
+    print(f"case d64_infinite {heads} routed={routed} {dtype}", flush=True)
+    H, Hkv = heads
+    n, d, front, window, key = 2000, 64, 16, 300, 900
+    q, k, v = (_rand((x, n, d), s, dtype).to(dev) for x, s in ((H, 61), (Hkv, 62), (Hkv, 63)))
+    idx = torch.empty(H, 1, 0, dtype=torch.int32, device=dev)
+    if routed:  # usable keys before and after `key` in one batch of every list
+        idx = torch.cat([torch.arange(40, 900, 20), torch.tensor([key]), torch.arange(1000, 1400, 25)]).int()
+        idx = idx.expand(H, 1, -1).contiguous().to(dev)
+    kw = dict(front=front, window=window, num_heads=H, kv_groups=H // Hkv, scale=d ** -0.5)
+    want = bigger_bird_flash(q, k, v, idx, **kw)
+    v = v.clone()
+    v[:, key, 7] = float("inf")
+    got = bigger_bird_flash(q, k, v, idx, **kw)
+    far = key // 64 * 64 - 31
+    assert torch.equal(got[:, :far], want[:, :far])
+    if not routed:
+        past = key + window + 64 + 32
+        assert torch.equal(got[:, past:], want[:, past:])
+    assert torch.isposinf(got[:, key + 40: key + 200, 7]).all() if not routed else torch.isposinf(got[:, 1700:, 7]).all()
+    other = torch.arange(d, device=dev) != 7
+    assert torch.equal(got[..., other], want[..., other])
+
+
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float16, 64)])
 def test_split_chunks_infinite_value(dtype, d, dev):
     """An infinite value in the first key chunk reaches its column as infinity and leaves the others alone: the merge
